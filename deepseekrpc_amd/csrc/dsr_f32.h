@@ -338,7 +338,7 @@ __device__ __forceinline__ int f32_sorted_tail(const RowSpec& r, F32Lists& t, Ge
 }
 
 // The 16-bit prefix of the k-th largest of the 16-bit key prefixes that the
-// workgroup's threads hold (NV each, val(0 .. NV-1); 0 is not counted), D
+// workgroup's threads hold (each(f) calls f for every one of a thread's; 0 is not counted), D
 // the largest of them; 0 when fewer than k are counted.  By distance d = D -
 // prefix: a coarse histogram of d / 8 over d < 2,048 (sixteen binades below a
 // positive maximum), then a fine one of d % 8 inside the selected coarse bin.
@@ -348,8 +348,8 @@ __device__ __forceinline__ int f32_sorted_tail(const RowSpec& r, F32Lists& t, Ge
 // fewer than k prefixes inside that distance take two 8-bit radix passes
 // over the whole prefix instead.  Each wave counts into its own histogram,
 // cleared by itself.  Every thread calls it.
-template <int NV, class Val>
-__device__ __forceinline__ uint32_t f32_tau16(F32Lists& t, int wave, int lane, uint32_t D, long long k, Val val) {
+template <class Each>
+__device__ __forceinline__ uint32_t f32_tau16_each(F32Lists& t, int wave, int lane, uint32_t D, long long k, Each each) {
   auto clear_hist = [&]() {
     *reinterpret_cast<uint4*>(&t.hist[wave][4 * lane]) = make_uint4(0u, 0u, 0u, 0u);
     wave_lds_sync();
@@ -360,16 +360,14 @@ __device__ __forceinline__ uint32_t f32_tau16(F32Lists& t, int wave, int lane, u
     uint32_t cbin = 0u;  // selected coarse bin (d / 8)
     for (int pass = 0; pass < 2; ++pass) {
       clear_hist();
-#pragma unroll
-      for (int i = 0; i < NV; ++i) {
-        const uint32_t x = val(i);
+      each([&](uint32_t x) {
         const uint32_t d = D - x;  // x <= D
         if (pass == 0) {
           if (x != 0u && d < 8u * kF32Bins) atomicAdd(&t.hist[wave][kF32Bins - 1 - (d >> 3)], 1u);
         } else {
           if (x != 0u && (d >> 3) == cbin) atomicAdd(&t.hist[wave][kF32Bins - 1 - (d & 7u)], 1u);
         }
-      }
+      });
       __syncthreads();
       long long above;
       const int b = f32_pick(t, rem, above);  // uniform
@@ -385,12 +383,11 @@ __device__ __forceinline__ uint32_t f32_tau16(F32Lists& t, int wave, int lane, u
     for (int pass = 0; pass < 2; ++pass) {
       const int shift = pass == 0 ? 24 : 16;
       clear_hist();
-#pragma unroll
-      for (int i = 0; i < NV; ++i) {
-        const uint32_t x = val(i) << 16;
+      each([&](uint32_t v) {
+        const uint32_t x = v << 16;
         const bool cnt = x != 0u && (pass == 0 || (x >> 24) == (prefix >> 24));
         if (cnt) atomicAdd(&t.hist[wave][(x >> shift) & 0xFFu], 1u);
-      }
+      });
       __syncthreads();
       long long above;
       const int b = f32_pick(t, rem, above);
@@ -401,6 +398,14 @@ __device__ __forceinline__ uint32_t f32_tau16(F32Lists& t, int wave, int lane, u
     tau16 = prefix >> 16;
   }
   return tau16;
+}
+
+template <int NV, class Val>
+__device__ __forceinline__ uint32_t f32_tau16(F32Lists& t, int wave, int lane, uint32_t D, long long k, Val val) {
+  return f32_tau16_each(t, wave, lane, D, k, [&](auto f) {
+#pragma unroll
+    for (int i = 0; i < NV; ++i) f(val(i));
+  });
 }
 
 constexpr int kDecided = -4;      // f32_list_finish: the row's outputs are written
@@ -544,39 +549,15 @@ __device__ __forceinline__ void f32_wave_tail(const dsr_sample_args_t& a, int64_
   }
 }
 
-// From the per-wave token lists (t.lv / t.li, wn entries in this wave) to
-// the row's decision: the row-wide list as float64 z = (v - max) / T, then
-// f32_sorted_tail, or radix_top_k and filter_tail when a bucket is too full.
-__device__ __forceinline__ int f32_list_finish(const dsr_sample_args_t& a, int64_t row, const RowSpec& r,
-                                               F32Shared& shu, int wave, int lane, int wn, double M, long long k,
-                                               int64_t V, unsigned& flags, DistOut& out, int64_t& n, int& why) {
+// Decides a row from its candidate list (t.cz / t.cid, nc entries, index
+// order): one wave's tail, the sorted tail, or radix_top_k and filter_tail
+// when a bucket is too full.
+__device__ __forceinline__ int f32_list_decide(const dsr_sample_args_t& a, int64_t row, const RowSpec& r, F32Shared& shu,
+                                               int64_t nc, long long k, int64_t V, unsigned& flags, DistOut& out,
+                                               int64_t& n, int& why) {
   F32Lists& t = shu.t;
   GenShared& sh = shu.gen;
   const int tid = threadIdx.x;
-  const dsr_policy_t& p = r.pol;
-  if (lane == 0) t.wn[wave] = wn;
-  __syncthreads();
-  int base = 0, total = 0, over = 0;
-#pragma unroll
-  for (int w = 0; w < kWaves; ++w) {
-    const int c = t.wn[w];
-    over |= c > kF32WaveCap ? 1 : 0;
-    if (w < wave) base += c;
-    total += c;
-  }
-  if (over) {
-    why = kHandCapacity;
-    return -1;
-  }
-  // The row-wide list in index order, as float64 (v - max) / T
-  // (sampling.py:86-88, true division).
-  const double T = p.temperature;
-  for (int i = lane; i < wn; i += 64) {
-    t.cz[base + i] = ((double)t.lv[wave][i] - M) / T;
-    t.cid[base + i] = t.li[wave][i];
-  }
-  __syncthreads();
-  const int64_t nc = total;
   if (nc <= kWaveTailMax) {
     f32_wave_tail(a, row, r, t, (int)nc, k, V, flags);
     return kDecided;
@@ -618,6 +599,41 @@ __device__ __forceinline__ int f32_list_finish(const dsr_sample_args_t& a, int64
   n = nk;
   const int32_t* kid = t.kid;
   return filter_tail(r, t.kz, nk, V, false, 0, -1, sh, flags, out, [kid](int64_t j) { return (int64_t)kid[j]; });
+}
+
+// From the per-wave token lists (t.lv / t.li, wn entries in this wave) to
+// the row's decision: the row-wide list as float64 z = (v - max) / T, then
+// f32_sorted_tail, or radix_top_k and filter_tail when a bucket is too full.
+__device__ __forceinline__ int f32_list_finish(const dsr_sample_args_t& a, int64_t row, const RowSpec& r,
+                                               F32Shared& shu, int wave, int lane, int wn, double M, long long k,
+                                               int64_t V, unsigned& flags, DistOut& out, int64_t& n, int& why) {
+  F32Lists& t = shu.t;
+  GenShared& sh = shu.gen;
+  const int tid = threadIdx.x;
+  const dsr_policy_t& p = r.pol;
+  if (lane == 0) t.wn[wave] = wn;
+  __syncthreads();
+  int base = 0, total = 0, over = 0;
+#pragma unroll
+  for (int w = 0; w < kWaves; ++w) {
+    const int c = t.wn[w];
+    over |= c > kF32WaveCap ? 1 : 0;
+    if (w < wave) base += c;
+    total += c;
+  }
+  if (over) {
+    why = kHandCapacity;
+    return -1;
+  }
+  // The row-wide list in index order, as float64 (v - max) / T
+  // (sampling.py:86-88, true division).
+  const double T = p.temperature;
+  for (int i = lane; i < wn; i += 64) {
+    t.cz[base + i] = ((double)t.lv[wave][i] - M) / T;
+    t.cid[base + i] = t.li[wave][i];
+  }
+  __syncthreads();
+  return f32_list_decide(a, row, r, shu, total, k, V, flags, out, n, why);
 }
 
 // Returns a status when the row is decided (kz / kid then hold the n final

@@ -31,6 +31,7 @@
 #include "dsr_numpy.h"
 #include "dsr_split.h"
 #include "dsr_verify.h"
+#include "dsr_wide.h"
 
 namespace dsr {
 
@@ -250,6 +251,149 @@ __global__ __launch_bounds__(kThreads) void k_sample_bf16_full(dsr_sample_args_t
   DistOut d;
   int st = general_distribution(r, sh.g, flags, d);
   finish_row<RNG>(a, row, W, a.vocab, st, d, flags, sh.g);
+}
+
+// Sliced path, step three (dsr_wide.h): one workgroup finishes a row from
+// its slices' records, or redoes it on the general path.  Two kernels, each
+// leaving the other's rows untouched (the hints say which are needed):
+// k_wide_topk takes top-k rows and, `others`, greedy rows and rows outside
+// the path's limits; k_wide_draw takes whole rows and always the greedy and
+// outside ones.  `mark` is the path flag of the rows decided here.
+template <class Src>
+__device__ __forceinline__ void wide_greedy(const Src& src, int64_t row, const RowSpec& r, const WideRow& w, bool draws,
+                                            unsigned mark) {
+  if (threadIdx.x != 0) return;  // sampling.py:82-85: the first index of the maximum
+  if (r.probs_f32) r.probs_f32[w.first] = 1.0f;
+  if (r.probs_f64) r.probs_f64[w.first] = 1.0;
+  if (r.kept_bits) r.kept_bits[w.first >> 5] = 1u << (w.first & 31);
+  fast_write_result(src.a, row, DSR_OK, draws ? w.first : -1, 0, mark);
+  src.onehot(row, w.first);
+}
+
+// The general path for a row this path hands over.
+template <class Src, bool RNG>
+__device__ __forceinline__ void wide_general(const Src& src, int64_t row, const RowSpec& r, int why, GenShared& sh) {
+  __syncthreads();  // every thread is done with the row's records and lists
+  unsigned flags = DSR_FLAG_GENERAL | ((unsigned)why << 4);
+  DistOut d;
+  const int st = general_distribution(r, sh, flags, d);
+  finish_row<RNG>(src.a, row, r.W, r.V, st, d, flags, sh);
+}
+
+template <class Src, int DT, bool RNG>
+__global__ __launch_bounds__(kThreads) void k_wide_topk(Src src, int others, unsigned mark) {
+  __shared__ F32Shared sh;
+  const int64_t row = blockIdx.x;
+  if (!src.takes(row)) return;
+  const RowSpec r = src.spec(row);
+  char* ws = src.ws(row);
+  const WideLayout L(r.V);
+  const WideKind kind = wide_kind(r, L);
+  if (kind != kWideTopK && !others) return;
+  int why = 0;
+  unsigned flags = mark;
+  DistOut d;
+  d.onehot = -1;
+  d.npos = 0;
+  d.first = -1;
+  int64_t n = 0;
+  int st = -1;
+  if (kind == kWideTopK || kind == kWideGreedy) {
+    double f;
+    const WideRow w = wide_row_of<false>(L, ws, r, nullptr, f);
+    if (w.bad) {
+      why = kHandInvalid;
+    } else if (kind == kWideGreedy) {
+      wide_greedy(src, row, r, w, has_draws<RNG>(src.a), mark);
+      return;
+    } else {
+      const int nc = wide_candidates<DT>(r, L, ws, w.M, r.pol.top_k, sh, why);
+      if (nc >= 0) st = f32_list_decide(src.a, row, r, sh, nc, r.pol.top_k, r.V, flags, d, n, why);
+    }
+  } else {
+    why = wide_outside(r);
+  }
+  if (st == kDecided) return;
+  if (st >= 0) {
+    const int32_t* kid = sh.t.kid;
+    finish_row<RNG>(src.a, row, sh.t.kz, n, st, d, flags, sh.gen, [kid](int64_t j) { return (int64_t)kid[j]; });
+    return;
+  }
+  wide_general<Src, RNG>(src, row, r, why, sh.gen);
+}
+
+template <class Src, int DT, bool RNG>
+__global__ __launch_bounds__(kThreads) void k_wide_draw(Src src, unsigned mark) {
+  __shared__ WideDrawShared sh;
+  const int64_t row = blockIdx.x;
+  if (!src.takes(row)) return;
+  const dsr_sample_args_t& a = src.a;
+  const RowSpec r = src.spec(row);
+  char* ws = src.ws(row);
+  const WideLayout L(r.V);
+  const WideKind kind = wide_kind(r, L);
+  if (kind == kWideTopK) return;
+  const int tid = threadIdx.x;
+  int why = 0;
+  if (kind == kWideNone) {
+    why = wide_outside(r);
+  } else {
+    const WideRow w = *L.row(ws);
+    if (w.bad) {
+      why = kHandInvalid;
+    } else if (kind == kWideGreedy) {
+      wide_greedy(src, row, r, w, has_draws<RNG>(a), mark);
+      return;
+    } else if (wide_nofilter(r.pol) && r.pen_n > 0 && (wide_neutral(r.pol) || 2 * w.crowded > L.nS)) {
+      // No filter: a table that only the count check reads, and rows whose
+      // tokens crowd into one block (the full-vocabulary kernel's key counts
+      // overflow on them), stay with the general path.
+      why = kHandCapacity;
+    } else {
+      exp_table_init(sh.etab);
+      if (tid == 0) sh.close = 0u;
+      lds_barrier();
+      unsigned flags = mark;
+      double Sk = 0.0, vc = -INFINITY;
+      int32_t ic = INT32_MAX;
+      long long npos = 0;
+      const WideKeep every{w.M, r.pol.temperature, -INFINITY, r.pol.min_p, INT32_MAX, sh.etab};
+      why = wide_whole(r, L, ws, w, sh, every, vc, ic, Sk, npos, flags);
+      if (why == 0) {
+        int st = Sk > 0.0 ? DSR_OK : DSR_E_NO_MASS;
+        int64_t token = -1;
+        int used = 0;
+        if (st == DSR_OK && has_draws<RNG>(a)) {
+          const WideKeep K{w.M, r.pol.temperature, vc, r.pol.min_p, ic, sh.etab};
+          if (npos == 1) {  // sampling.py:120-122: the single positive token; no uniform is drawn
+            unsigned none = 0u;
+            token = wide_walk<DT>(r, L, ws, sh, K, Sk, npos, 0.0, none);
+          } else {
+            uint64_t next[4];
+            const double u = RNG ? pcg64_random(a.rng_state + 4 * row, next) : a.uniforms[row];
+            if (!(u >= 0.0 && u < 1.0)) {
+              st = DSR_E_UNIFORM;
+            } else {
+              token = wide_walk<DT>(r, L, ws, sh, K, Sk, npos, u, flags);
+              used = 1;
+            }
+            if (RNG) {
+              __syncthreads();  // every thread has read the state
+              if (tid == 0) store_rng(a, row, next);
+            }
+          }
+        }
+        if (tid == 0) {
+          fast_write_result(a, row, st, token, used, flags);
+          *L.dec(ws) = WideDec{Sk, vc, ic, 0};
+        }
+        return;
+      }
+    }
+  }
+  wide_general<Src, RNG>(src, row, r, why, sh.g);
+  __syncthreads();  // the row's workspace is free again
+  if (tid == 0) L.dec(ws)->done = 1;  // its outputs are complete
 }
 
 // ---------------------------------------------------------------------------
@@ -867,6 +1011,57 @@ using namespace dsr;
 
 static int32_t launched() { return hipGetLastError() == hipSuccess ? 0 : DSR_ERR_LAUNCH; }
 
+// FP32 top-k batches of at most this many 8,192-token slices run on the
+// sliced path instead of k_sample_f32: 16 slices of one row shorten its read
+// (V = 129,280, top-k 50: 18.6 us against 26.3 for 1 row, 21.7 against 27.9 for
+// 32; V = 40,000, 64 rows: 21.7 against 26.7), until the rows alone fill the chip (256 rows:
+// 42.7 against 40.4; top-k up to 1,024 with a mask, 16 rows: 40.9 against 42.1,
+// 64 rows: 46.6 against 43.2).  From 32,768 tokens on: a shorter row has too
+// few 16-token groups for every top-k up to 1,024.
+constexpr int64_t kWideTopkSlices = 512;
+constexpr int64_t kWideTopkVocab = 32768;
+
+// The sliced path takes batches whose policies the caller describes (its
+// hints leave out the launches no row needs).  Against the split path and the
+// general one (V = 129,280): FP32 rows of mixed whole policies, 1 row 25.9 us against
+// 112, 64 rows 72 against 308, 256 rows 146 against 511; FP32 top-k 50 with
+// 2,000-token histories, 1 row 22.6 against 46.5, 64 rows 31.6 against 98.7.
+static bool wide_path_eligible(const dsr_sample_args_t& a) {
+  return (a.dtype == DSR_BF16 || a.dtype == DSR_F32) && a.vocab >= kWideMinVocab && a.rows > 0 &&
+         (a.hints & (DSR_HINT_WHOLE_SOME | DSR_HINT_WHOLE_ALL | DSR_HINT_TOPK_ALL)) &&
+         a.rows * (int64_t)WideLayout(a.vocab).nS * kWideThreads < ((int64_t)1 << 32);
+}
+
+template <class Src, int DT, bool RNG>
+static void wide_launch(const Src& src, int64_t rows, uint32_t hints, bool probs, unsigned mark, hipStream_t s) {
+  const int nS = WideLayout(src.a.vocab).nS;
+  const dim3 slices((unsigned)(rows * nS)), whole((unsigned)rows);
+  const bool topk_only = hints & DSR_HINT_TOPK_ALL, whole_only = hints & DSR_HINT_WHOLE_ALL;
+  const int later = probs && !topk_only;
+  if (topk_only) hipLaunchKernelGGL((k_wide_scan<Src, DT, false>), slices, dim3(kWideThreads), 0, s, src, nS, later);
+  else hipLaunchKernelGGL((k_wide_scan<Src, DT, true>), slices, dim3(kWideThreads), 0, s, src, nS, later);
+  if (!topk_only) {
+    hipLaunchKernelGGL((k_wide_bracket<Src>), whole, dim3(kBracketThreads), 0, s, src);
+    hipLaunchKernelGGL((k_wide_collect<Src, DT>), slices, dim3(kWideThreads), 0, s, src, nS);
+    hipLaunchKernelGGL((k_wide_draw<Src, DT, RNG>), whole, dim3(kThreads), 0, s, src, mark);
+  }
+  if (!whole_only)
+    hipLaunchKernelGGL((k_wide_topk<Src, DT, RNG>), whole, dim3(kThreads), 0, s, src, topk_only ? 1 : 0, mark);
+  if (later) hipLaunchKernelGGL((k_wide_probs<Src, DT>), slices, dim3(kWideThreads), 0, s, src, nS);
+}
+
+static void wide_sample(const dsr_sample_args_t& a, unsigned mark, hipStream_t s) {
+  const WideSampleRows src{a};
+  const bool probs = a.out_probs_f32 || a.out_probs_f64, rng = a.rng_state != nullptr;
+  if (a.dtype == DSR_BF16) {
+    if (rng) wide_launch<WideSampleRows, DSR_BF16, true>(src, a.rows, a.hints, probs, mark, s);
+    else wide_launch<WideSampleRows, DSR_BF16, false>(src, a.rows, a.hints, probs, mark, s);
+  } else {
+    if (rng) wide_launch<WideSampleRows, DSR_F32, true>(src, a.rows, a.hints, probs, mark, s);
+    else wide_launch<WideSampleRows, DSR_F32, false>(src, a.rows, a.hints, probs, mark, s);
+  }
+}
+
 extern "C" {
 
 int32_t dsr_abi_version(void) { return DSR_ABI_VERSION; }
@@ -948,6 +1143,7 @@ static int32_t sample_rows(const dsr_sample_args_t* args, const dsr_head_part_t*
     if (k.rng_state) hipLaunchKernelGGL(k_sample_bf16_full<true>, grid, dim3(kThreads), 0, s, k);
     else hipLaunchKernelGGL(k_sample_bf16_full<false>, grid, dim3(kThreads), 0, s, k);
   };
+  const bool wide = wide_path_eligible(a);
   if (fast_path_eligible(a)) {
     // A bf16 batch with no history or bias: whole rows (no top-k register
     // cut) go to the full-vocabulary kernel when the caller says it has some.
@@ -959,9 +1155,14 @@ static int32_t sample_rows(const dsr_sample_args_t* args, const dsr_head_part_t*
     } else {
       launch_fast(0u);
     }
-  } else if (full_path_eligible(a)) {
+  } else if (full_path_eligible(a) && !(wide && (a.hints & DSR_HINT_TOPK_ALL))) {
+    // bf16 rows with a history and no top-k: one workgroup per row keeps the
+    // row in registers (64 rows with 4,096-token histories: 73 us, against 98
+    // on the sliced path; 1 row: 68 against 72).  It has no top-k cut, and
+    // the general path takes about 1 ms for such rows: batches of top-k rows
+    // go to the sliced path (64 rows, top-k 50: 32 us).
     launch_full(0u);
-  } else if (f32_path_eligible(a)) {
+  } else if (f32_path_eligible(a) && !(wide && !parts && a.vocab >= kWideTopkVocab && a.rows * WideLayout(a.vocab).nS <= kWideTopkSlices)) {
     if (a.out_probs_f32 || a.out_probs_f64) {
       const int64_t chunks = (a.vocab + kZeroChunk - 1) / kZeroChunk;
       hipLaunchKernelGGL(k_zero_probs, dim3((unsigned)(a.rows * chunks)), dim3(kZeroThreads), 0, s, a.out_probs_f32,
@@ -970,6 +1171,8 @@ static int32_t sample_rows(const dsr_sample_args_t* args, const dsr_head_part_t*
     const dsr_head_part_t* hp = parts && f32_head_eligible(a) ? parts : nullptr;
     if (a.rng_state) hipLaunchKernelGGL(k_sample_f32<true>, dim3((unsigned)a.rows), dim3(kThreads), 0, s, a, hp);
     else hipLaunchKernelGGL(k_sample_f32<false>, dim3((unsigned)a.rows), dim3(kThreads), 0, s, a, hp);
+  } else if (wide) {
+    wide_sample(a, f32_path_eligible(a) ? DSR_FLAG_F32_TOPK : DSR_FLAG_SPLIT, s);
   } else if (split_path_eligible(a)) {
     const int smax = split_max_slices(a.rows);
     hipLaunchKernelGGL(k_split_select, dim3((unsigned)(a.rows * smax)), dim3(kThreads), 0, s, a, smax);

@@ -77,12 +77,11 @@ extern "C" {
 #define DSR_FLAG_MARGIN 1u      /* a threshold decision sat inside the rounding band */
 #define DSR_FLAG_GENERAL 2u     /* decided by the general (workspace) path; bits 4-7 give
                                    the reason a row left a faster path */
-#define DSR_FLAG_SPLIT 4u       /* decided from per-slice candidates (rows split over several
-                                   workgroups: top-k <= 1024, greedy, top-p / min-p whose
-                                   kept set lies among the row's 512 largest values, or no
-                                   filter with no history or bias) */
-#define DSR_FLAG_F32_TOPK 8u    /* decided by the one-workgroup FP32 top-k path (greedy or
-                                   1 <= top-k <= 1024, no history or bias) */
+#define DSR_FLAG_SPLIT 4u       /* decided from per-slice records (rows split over several
+                                   workgroups: top-k <= 1024, greedy, top-p / min-p, or no
+                                   filter) */
+#define DSR_FLAG_F32_TOPK 8u    /* decided by the FP32 top-k path (greedy or 1 <= top-k <= 1024,
+                                   no history or bias) */
 
 /* Kernel-choice hints (dsr_sample_args_t.hints, dsr_verify_args_t.hints):
  * statements about the batch's policies that let the library choose its
@@ -100,8 +99,11 @@ extern "C" {
  * DSR_HINT_TOPK_ALL: every row's policy is in bounds and is greedy or has
  *   1 <= top_k <= 1024 below the vocabulary; an FP32 batch with no history
  *   or bias (rows 16-byte aligned, vocab a multiple of 4, at most 131,072)
- *   then runs the one-workgroup FP32 top-k kernel.  Like the WHOLE hints it
- *   changes no result.
+ *   then runs the FP32 top-k path (one workgroup per row, or the row in
+ *   slices for small batches).  Like the WHOLE hints it changes no result.
+ * Any of the three lets FP32 batches, and bf16 batches that the register
+ *   kernels cannot take (a bias, unaligned rows, top-k with a history), run
+ *   in 8,192-token slices over the whole chip.
  * DSR_HINT_VERIFY_FAST: a promise that every request has a policy with no
  *   filter (top_k 0 or >= vocab, top_p 1, min_p 0) and that the call passes
  *   no history, bias or allow mask, so the launch that builds general-path
