@@ -156,6 +156,22 @@ def verify_hints(arr: np.ndarray | None, vocab: int, plain: bool) -> int:
     return N.HINT_VERIFY_FAST if ok.all() else 0
 
 
+def _verify_call_hints(arr: np.ndarray | None, vocab: int, plain: bool) -> int:
+    """``verify_hints``, and for requests on the sliced path: DSR_HINT_TOPK_ALL
+    when every one cuts to a top-k it lists (or is greedy, where the call has
+    no fast path), DSR_HINT_WHOLE_SOME on a plain call whose requests all have
+    a filter it takes.  These two only choose launches."""
+    hints = verify_hints(arr, vocab, plain)
+    if hints or arr is None or len(arr) == 0:
+        return hints
+    k, ok = arr["top_k"], policies_in_bounds(arr)
+    cut = ok & (k >= 1) & (k <= FAST_MAX_K) & (k < vocab)
+    if (cut | (ok & (not plain) & (arr["temperature"] == 0))).all():
+        return N.HINT_TOPK_ALL
+    filtered = ok & ((k == 0) | (k >= vocab)) & ((arr["top_p"] < 1.0) | (arr["min_p"] != 0.0))
+    return N.HINT_WHOLE_SOME if plain and (cut | filtered).all() else 0
+
+
 @dataclass
 class HistoryTable:
     """Per-row sparse token-history counts in CSR form (device tensors).
@@ -805,7 +821,7 @@ def verify_drafts(target: torch.Tensor, draft: torch.Tensor, draft_ids: torch.Te
     (int64 ``[rows, 4]``, see ``pcg64_states``) instead draw them on the
     device from each request's accept / target PCG64 state, which is advanced
     by exactly the draws the decision uses.  ``hints`` overrides the
-    DSR_HINT_VERIFY_FAST bit derived from the policies.  ``head`` =
+    DSR_HINT_* bits derived from the policies.  ``head`` =
     ``(target, draft)`` ``HeadResult`` s of the ``vocab_head`` calls that
     wrote ``target`` and ``draft``: the per-row statistics then come from
     their records (``dsr_verify_drafts_head``).
@@ -854,8 +870,8 @@ def verify_drafts(target: torch.Tensor, draft: torch.Tensor, draft_ids: torch.Te
     if allow_bits is not None:
         _require_cuda(allow_bits, "allow_bits")
         a.allow_bits, a.allow_ld = allow_bits.data_ptr(), allow_bits.shape[-1]
-    a.hints = verify_hints(getattr(policies, "dsr_policies", None), V,
-                           not _nonempty(history, "ids") and not _nonempty(bias, "ids") and allow_bits is None) \
+    a.hints = _verify_call_hints(getattr(policies, "dsr_policies", None), V,
+                                 not _nonempty(history, "ids") and not _nonempty(bias, "ids") and allow_bits is None) \
         if hints is None else hints
     a.u_accept = u_accept.data_ptr() if K > 0 and u_accept is not None else None
     a.u_target = u_target.data_ptr() if u_target is not None else None

@@ -89,7 +89,21 @@ struct VerifyLayout {
   int64_t rows;
   int fast_inputs;   // no history, bias or allow mask
   int dists_built;   // k_verify_dists ran before k_verify_chain
+  int wide;          // the requests go through the sliced path first
 };
+
+// What the sliced path left for a distribution (info[3]): nothing (the
+// distribution is built in full), a one-hot index, a list of kept tokens, or
+// a kept set.
+enum WideForm { kFormDense = 0, kFormOne = 1, kFormList = 2, kFormWhole = 3 };
+
+// Whether every distribution of request `row` was decided there (uniform).
+__device__ __forceinline__ bool wide_request(const VerifyLayout& L, int64_t row) {
+  const int32_t* info = L.info + row * L.slots * 4;
+  bool all = true;
+  for (int s = 0; s < (int)L.slots; ++s) all = all && info[s * 4 + 3] != kFormDense;
+  return all;
+}
 
 __host__ __device__ inline size_t verify_ws_bytes(int64_t rows, int32_t K, int64_t V) {
   const size_t slots = (size_t)(2 * K + 1);
@@ -124,6 +138,7 @@ __host__ inline VerifyLayout verify_layout(void* ws, int64_t rows, int32_t K, in
   L.rows = rows;
   L.fast_inputs = 0;
   L.dists_built = 1;
+  L.wide = 0;
   return L;
 }
 
@@ -191,10 +206,8 @@ __device__ __forceinline__ Request request_of(const A& a, int64_t row) {
 // ---------------------------------------------------------------------------
 // General path.
 
-// Distribution `slot` of general-path request `row`, built in full into its
-// workspace row, its status / one-hot / flags into L.info.
-__device__ __forceinline__ void verify_build_dist(const dsr_verify_args_t& a, const VerifyLayout& L, int64_t row, int slot,
-                                  GenShared& sh) {
+// Distribution `slot` of request `row`, with the drafts before it as its prefix.
+__device__ __forceinline__ RowSpec verify_row_spec(const dsr_verify_args_t& a, const VerifyLayout& L, int64_t row, int slot) {
   const int K = a.K;
   const bool is_target = slot <= K;
   const int j = is_target ? slot : slot - (K + 1);
@@ -229,6 +242,14 @@ __device__ __forceinline__ void verify_build_dist(const dsr_verify_args_t& a, co
   r.kept_words = 0;
   r.probs_f32 = nullptr;
   r.probs_f64 = nullptr;
+  return r;
+}
+
+// A general-path request's distribution, built in full into its workspace
+// row, its status / one-hot / flags into L.info.
+__device__ __forceinline__ void verify_build_dist(const dsr_verify_args_t& a, const VerifyLayout& L, int64_t row, int slot,
+                                  GenShared& sh) {
+  const RowSpec r = verify_row_spec(a, L, row, slot);
   unsigned flags = 0;
   DistOut d;
   int st = general_distribution(r, sh, flags, d);
@@ -240,12 +261,14 @@ __device__ __forceinline__ void verify_build_dist(const dsr_verify_args_t& a, co
   }
 }
 
-// One workgroup per distribution of every general-path request.
+// One workgroup per distribution of every general-path request the sliced
+// path did not decide.
 __global__ __launch_bounds__(kThreads) void k_verify_dists(dsr_verify_args_t a, VerifyLayout L) {
   __shared__ GenShared sh;
   const int64_t row = blockIdx.x / L.slots;
   const int slot = (int)(blockIdx.x % L.slots);
   if (verify_fast_row(a, L, row)) return;
+  if (L.wide && wide_request(L, row)) return;
   verify_build_dist(a, L, row, slot, sh);
 }
 

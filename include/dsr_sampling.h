@@ -104,6 +104,11 @@ extern "C" {
  * Any of the three lets FP32 batches, and bf16 batches that the register
  *   kernels cannot take (a bias, unaligned rows, top-k with a history), run
  *   in 8,192-token slices over the whole chip.
+ *   A verifier call with no history, bias or allow mask runs its requests in
+ *   such slices when any of the three is given (best when every request has a
+ *   filter); one with them always does, and DSR_HINT_TOPK_ALL leaves out the
+ *   launches that other requests need.  A request that contradicts a hint is
+ *   still decided exactly.
  * DSR_HINT_VERIFY_FAST: a promise that every request has a policy with no
  *   filter (top_k 0 or >= vocab, top_p 1, min_p 0) and that the call passes
  *   no history, bias or allow mask, so the launch that builds general-path
