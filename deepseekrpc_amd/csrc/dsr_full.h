@@ -420,8 +420,8 @@ __device__ __forceinline__ int full_sample_row(const dsr_sample_args_t& a, int64
   // One barrier for the key maximum (with the invalid flag), one more for
   // the history's count total and value maximum when the row has a history
   // (pn is uniform).
-  const uint32_t red = bs.max((kmx << 1) | badv);
-  const uint32_t Mk = red >> 1;
+  const uint32_t red = bs.max((badv << 16) | kmx);  // a bad thread's word is above every key
+  const uint32_t Mk = red & 0xFFFFu;
   long long csum_all = 0;
   double PM = -(double)INFINITY;
   if (pn > 0) {
@@ -429,7 +429,7 @@ __device__ __forceinline__ int full_sample_row(const dsr_sample_args_t& a, int64
     PM = pmax;
     bs.sum_max(csum_all, PM);
   }
-  if ((red & 1u) || csum_all > DSR_MAX_COUNT) return kHandInvalid;
+  if ((red >> 16) || csum_all > DSR_MAX_COUNT) return kHandInvalid;
   const double Mv = Mk > kKeyNegInf ? bf16_key_value(Mk) : -(double)INFINITY;
   const double M = Mv > PM ? Mv : PM;
   if (!(M > -(double)INFINITY)) return kHandInvalid;  // every token masked or -inf: reported by the general path

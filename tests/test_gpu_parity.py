@@ -448,3 +448,22 @@ def test_verify_golden_on_gpu(case):
         case["accepted"], case["output_ids"], case["pending"], case["stop"])
     assert int(res.used_accept.item()) == case["calls"].count("accept")
     assert int(res.used_target.item()) == case["calls"].count("target")
+
+
+@pytest.mark.parametrize("temperature", [0.0, 1.0])
+def test_bad_logit_at_a_token_out_of_play(temperature):
+    """NaN or +inf at a penalised or a masked token still makes the row invalid
+    (sampling.py:50-52 reads the whole vector)."""
+    V = 520
+    rng = np.random.default_rng(9)
+    x = np.repeat(rng.normal(0, 1, (1, V)).astype(np.float32), 5, 0)
+    x[:, 17] = 8.0
+    x[0, 300] = x[1, 301] = np.nan
+    x[2, 300] = x[3, 301] = np.inf
+    allowed = np.ones((5, V), bool)
+    allowed[:, 301] = False
+    bits = torch.from_numpy(batch.pack_allow(allowed).view(np.int32)).cuda()
+    table = batch.HistoryTable.from_token_lists([[300, 400]] * 5, device="cuda")
+    got = batch.sample_rows(torch.from_numpy(x).to(torch.bfloat16).cuda(), [dict(temperature=temperature, presence_penalty=0.5)] * 5,
+                            uniforms=torch.zeros(5, dtype=torch.float64, device="cuda"), history=table, allow_bits=bits)
+    assert got.status.tolist() == [N.E_LOGITS] * 4 + [0]
