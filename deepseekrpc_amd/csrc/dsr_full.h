@@ -449,7 +449,7 @@ __device__ __forceinline__ int full_sample_row(const dsr_sample_args_t& a, int64
           if (key_at(d[j], e) == Mk) f = 8ll * c + e;
       }
     }
-    if (PM == M && pfirst < f) f = pfirst;
+    if (pmax == M && pfirst < f) f = pfirst;  // this thread's own entries
     return bs.min(f);
   };
   if (greedy) {

@@ -450,6 +450,23 @@ def test_verify_golden_on_gpu(case):
     assert int(res.used_target.item()) == case["calls"].count("target")
 
 
+@pytest.mark.parametrize("V", [520, 5000])
+def test_greedy_maximum_among_penalised_tokens(V):
+    """A greedy row whose maximum is a token of its history: its index, not the
+    first one of the history (sampling.py:82-85)."""
+    rng = np.random.default_rng(V)
+    x = rng.normal(0, 1, (4, V)).astype(np.float32)
+    hist = [np.sort(rng.choice(V, 40, replace=False)) for _ in range(4)]
+    best = [int(h[k]) for h, k in zip(hist, (39, 20, 3, 0))]
+    for r, b in enumerate(best):
+        x[r, b] = 9.0 + r
+    logits = torch.from_numpy(x).to(torch.bfloat16).cuda()
+    table = batch.HistoryTable.from_token_lists([h.tolist() for h in hist], device="cuda")
+    pol = dict(temperature=0.0, repetition_penalty=1.1, presence_penalty=0.5)
+    got = batch.sample_rows(logits, [pol] * 4, uniforms=torch.zeros(4, dtype=torch.float64, device="cuda"), history=table)
+    assert got.tokens.tolist() == best and (got.status == 0).all() and (got.flags == 0).all()
+
+
 @pytest.mark.parametrize("temperature", [0.0, 1.0])
 def test_bad_logit_at_a_token_out_of_play(temperature):
     """NaN or +inf at a penalised or a masked token still makes the row invalid
