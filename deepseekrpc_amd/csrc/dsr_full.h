@@ -1083,4 +1083,168 @@ __device__ __forceinline__ int full_sample_row(const dsr_sample_args_t& a, int64
   return sh.bc_i[2] ? kHandCapacity : 0;  // unreachable: thr lies inside the chunk found above
 }
 
+
+// Greedy rows with a history, in a launch of their own ahead of the
+// full-vocabulary kernel when a batch has more rows than the chip has CUs.  A
+// greedy row needs no key counts: 22 KB of LDS and 64 registers let two rows
+// share a CU, so one's loads hide the other's steps, where the
+// full-vocabulary kernel's 160 KB hold one; and the sampled rows, left alone
+// in that kernel, no longer wait in launch order behind greedy ones (the
+// workgroups go to XCDs and shader engines in turn, so a batch of alternating
+// rows kept the sampled ones on half of them).
+// 1,024 rows of 129,280 with 16,384-token histories, greedy and nearly flat
+// top-p rows in turn: 300 us with this launch and rotated rows (spread_row),
+// 378 with rotated rows alone, 459 with neither.
+constexpr int32_t kGreedyLeft = INT32_MIN;  // out_status of a greedy row left to the full-vocabulary kernel
+
+struct GreedyShared {
+  uint32_t pbits[kFastMaxVocab / 32];  // allowed tokens the history does not touch
+  uint32_t lut[256][4];                // allow byte -> disallowed masks
+  SyncSlots sync;
+};
+
+template <bool RNG>
+__device__ __forceinline__ bool greedy_row(const dsr_sample_args_t& a, int64_t row, const dsr_policy_t& pol, GreedyShared& sh) {
+  const int tid = threadIdx.x, lane = lane_id();
+  const int wave = __builtin_amdgcn_readfirstlane(wave_id());
+  const int64_t V = a.vocab;
+  const uint32_t C = (uint32_t)(V >> 3);
+  const uint32_t CW = (C + kWaves - 1) / kWaves;
+  const int64_t o0 = a.pen_off[row], pn = a.pen_off[row + 1] - o0;
+  // The full-vocabulary kernel's limits: it hands such rows over itself.
+  if (!policy_ok(pol) || (pol.top_k != 0 && pol.top_k < V) || pn < 0 || 2 * pn > (int64_t)((V + 31) & ~31)) return false;
+  BlockSync bs(sh.sync);
+  const uint32_t nwords = (uint32_t)((V + 31) >> 5);
+  const uint32_t* allow = a.allow_bits ? a.allow_bits + row * a.allow_ld : nullptr;
+  const __amdgpu_buffer_rsrc_t rrs = __builtin_amdgcn_make_buffer_rsrc(
+      (void*)((const uint16_t*)a.logits + row * a.ld), (short)0, (int)(V * 2), 0x00020000);
+  uint4 d[4];
+  auto chunk = [&](int j) -> uint4 {
+    const uint32_t cw = (uint32_t)j * 64u + (uint32_t)lane;
+    const auto v = __builtin_amdgcn_raw_buffer_load_b128(
+        rrs, (int)(cw < CW ? ((uint32_t)wave * CW + cw) * 16u : 0x7FFFFFF0u), 0, 0);
+    return make_uint4(v[0], v[1], v[2], v[3]);
+  };
+  {
+    const uint32_t m = (uint32_t)tid >> 2, q = (uint32_t)tid & 3u;
+    sh.lut[m][q] = (((m >> (2 * q)) & 1u) ? 0u : 0x0000FFFFu) | (((m >> (2 * q + 1)) & 1u) ? 0u : 0xFFFF0000u);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const uint32_t w = (uint32_t)tid + (uint32_t)i * kThreads;
+      if (w < kFastMaxVocab / 32) sh.pbits[w] = (allow && w < nwords) ? allow[w] : 0xFFFFFFFFu;
+    }
+  }
+  lds_barrier();
+
+  // The history: its tokens leave the bitmap, its adjusted values
+  // (sampling.py:59-66, then the mask :75-79) give a maximum and its first index.
+  int bad = 0;
+  long long csum = 0;
+  double pmax = -INFINITY;
+  long long pfirst = LLONG_MAX;
+  for (int64_t base = tid; base < pn; base += (int64_t)kPenBatch * kThreads) {
+    int32_t id[kPenBatch], prv[kPenBatch], c[kPenBatch], g[kPenBatch];
+#pragma unroll
+    for (int i = 0; i < kPenBatch; ++i) {
+      const int64_t e = base + (int64_t)i * kThreads;
+      const bool in = e < pn;
+      id[i] = in ? a.pen_ids[o0 + e] : 0;
+      prv[i] = (in && e > 0) ? a.pen_ids[o0 + e - 1] : INT_MIN;
+      c[i] = in ? a.pen_count[o0 + e] : 0;
+      g[i] = in ? a.pen_gen[o0 + e] : 0;
+    }
+    uint32_t raw[kPenBatch];
+    bool ok[kPenBatch];
+#pragma unroll
+    for (int i = 0; i < kPenBatch; ++i) {
+      const int64_t e = base + (int64_t)i * kThreads;
+      ok[i] = e < pn && id[i] >= 0 && id[i] < V && prv[i] < id[i] && c[i] >= 0 && c[i] <= DSR_MAX_COUNT &&
+              g[i] >= 0 && g[i] <= c[i];
+      raw[i] = __builtin_amdgcn_raw_buffer_load_b16(rrs, ok[i] ? 2 * id[i] : 0x7FFFFFF0, 0, 0);
+    }
+#pragma unroll
+    for (int i = 0; i < kPenBatch; ++i) {
+      const int64_t e = base + (int64_t)i * kThreads;
+      if (e >= pn) continue;
+      bad |= ok[i] ? 0 : 1;
+      csum += c[i];
+      if (!ok[i]) continue;
+      atomicAnd(&sh.pbits[id[i] >> 5], ~(1u << (id[i] & 31)));
+      double x = (double)__uint_as_float(raw[i] << 16);
+      if (c[i] > 0) x = x >= 0.0 ? x / pol.repetition_penalty : x * pol.repetition_penalty;
+      const double pen = pol.presence_penalty * (g[i] > 0 ? 1.0 : 0.0) + pol.frequency_penalty * (double)g[i];
+      const double v = x - pen;
+      if (v > pmax && allowed_bit(allow, id[i])) {  // ids increase with e: the first holder stays; NaN logits: the raw check
+        pmax = v;
+        pfirst = id[i];
+      }
+    }
+  }
+  lds_barrier();
+
+  // The row, four chunks in flight: raw NaN / +inf check, and the largest
+  // untouched key with the first chunk of this thread that holds it.
+  uint32_t vmax_s = 0x80008000u, vmax_u = 0u, best = 0u;
+  int bj = 0;
+  auto keys = [&](uint4 v, int j, uint32_t k[4]) {
+    const uint32_t cw = (uint32_t)j * 64u + (uint32_t)lane, c = (uint32_t)wave * CW + cw;
+    const bool live = cw < CW && c < C;
+    const uint32_t cc = live ? c : 0u;
+    const uint32_t stay = (sh.pbits[cc >> 2] >> ((cc & 3u) * 8u)) & (live ? 0xFFu : 0u);
+    const uint4 m = *(const uint4*)sh.lut[stay];
+    k[0] = bf16x2_keys(v.x | m.x);
+    k[1] = bf16x2_keys(v.y | m.y);
+    k[2] = bf16x2_keys(v.z | m.z);
+    k[3] = bf16x2_keys(v.w | m.w);
+  };
+#pragma unroll 1
+  for (int j0 = 0; j0 < kFastChunks; j0 += 4) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) d[q] = chunk(j0 + q);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const uint32_t w[4] = {d[q].x, d[q].y, d[q].z, d[q].w};
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        vmax_s = pk_max_i16(vmax_s, w[i]);
+        vmax_u = pk_max_u16(vmax_u, w[i]);
+      }
+      uint32_t k[4];
+      keys(d[q], j0 + q, k);
+      const uint32_t p = pk_max_u16(pk_max_u16(k[0], k[1]), pk_max_u16(k[2], k[3])), h = max(p & 0xFFFFu, p >> 16);
+      bj = h > best ? j0 + q : bj;
+      best = max(best, h);
+    }
+  }
+  const uint32_t badv = (max((int)(short)(vmax_s & 0xFFFFu), (int)(short)(vmax_s >> 16)) >= 0x7F80 ||
+                         max(vmax_u & 0xFFFFu, vmax_u >> 16) >= 0xFF81u || bad) ? 1u : 0u;
+  const uint32_t red = bs.max((badv << 16) | best), Mk = red & 0xFFFFu;  // a bad thread's word is above every key
+  double PM = pmax;
+  bs.sum_max(csum, PM);
+  if ((red >> 16) || csum > DSR_MAX_COUNT) return false;
+  const double Mv = Mk > kKeyNegInf ? bf16_key_value(Mk) : -(double)INFINITY;
+  const double M = Mv > PM ? Mv : PM;
+  if (!(M > -(double)INFINITY) || M == 0.0) return false;  // nothing to keep; +-0 tie by index
+  long long f = LLONG_MAX;
+  if (Mv == M && best == Mk) {
+    uint32_t k[4];
+    keys(chunk(bj), bj, k);
+    uint32_t e = 8u;
+#pragma unroll
+    for (int i = 3; i >= 0; --i) {
+      if ((k[i] >> 16) == Mk) e = 2u * i + 1u;
+      if ((k[i] & 0xFFFFu) == Mk) e = 2u * i;
+    }
+    f = 8ll * ((uint32_t)wave * CW + (uint32_t)bj * 64u + (uint32_t)lane) + e;
+  }
+  if (pmax == M && pfirst < f) f = pfirst;
+  const long long tok = bs.min(f);  // sampling.py:82-85: the first index of the maximum
+  if (a.out_probs_f32 || a.out_probs_f64 || a.out_kept_bits) {
+    fast_clear_outputs(a, row);
+    if (tid == 0) fast_scatter(a, row, tok, 1.0);
+  }
+  if (tid == 0) fast_write_result(a, row, DSR_OK, has_draws<RNG>(a) ? tok : -1, 0, 0);
+  return true;
+}
+
 }  // namespace dsr

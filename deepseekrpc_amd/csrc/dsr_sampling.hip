@@ -236,13 +236,23 @@ struct FullKernelShared {
   };
 };
 
+// The row of workgroup b.  Workgroups go to the eight XCDs in turn, and in each
+// to its four shader engines in turn, whatever those still hold: in a batch
+// whose rows alternate in kind, the costly rows would all meet on the same
+// engines.  So group k of 32 workgroups takes its 32 rows rotated by 11 k,
+// which keeps moving every bit of the row's number over the engines.
+__device__ __forceinline__ int64_t spread_row(uint32_t b, uint32_t rows) {
+  return (b | 31u) < rows ? (int64_t)((b & ~31u) | ((b + 11u * (b >> 5)) & 31u)) : (int64_t)b;
+}
+
 template <bool RNG>
 __global__ __launch_bounds__(kThreads) void k_sample_bf16_full(dsr_sample_args_t a) {
   __shared__ FullKernelShared sh;
-  const int64_t row = blockIdx.x;
+  const int64_t row = spread_row(blockIdx.x, gridDim.x);
   // After the top-k register kernel: only the rows it left (uniform; read
   // before the row's loads are issued, so other rows cost no HBM traffic).
   if ((a.hints & kModeOnlyWhole) && !whole_row(a.policy[row].temperature, a.policy[row].top_k, a.vocab)) return;
+  if ((a.hints & kModeGreedyDone) && a.policy[row].temperature == 0.0 && a.out_status[row] != kGreedyLeft) return;
   const int why = full_sample_row<RNG>(a, row, sh.f);
   if (why == 0) return;
   __syncthreads();
@@ -252,6 +262,15 @@ __global__ __launch_bounds__(kThreads) void k_sample_bf16_full(dsr_sample_args_t
   DistOut d;
   int st = general_distribution(r, sh.g, flags, d);
   finish_row<RNG>(a, row, W, a.vocab, st, d, flags, sh.g);
+}
+
+template <bool RNG>
+__global__ __launch_bounds__(kThreads, 8) void k_greedy_bf16(dsr_sample_args_t a) {
+  __shared__ GreedyShared sh;
+  const int64_t row = spread_row(blockIdx.x, gridDim.x);
+  const dsr_policy_t pol = a.policy[row];
+  if (!(pol.temperature == 0.0)) return;
+  if (!greedy_row<RNG>(a, row, pol, sh) && threadIdx.x == 0) a.out_status[row] = kGreedyLeft;
 }
 
 // Sliced path, step three (dsr_wide.h): one workgroup finishes a row from
@@ -1101,6 +1120,7 @@ size_t dsr_verify_workspace_bytes(int64_t rows, int32_t K, int64_t vocab) {
 
 // The DSR_HINT_* bits a caller may set; any other bit is rejected, so the
 // field can take new meanings later without an ABI change.
+constexpr int64_t kFullRows = 256;  // CUs: the full-vocabulary kernel holds one row on each
 static constexpr uint32_t kHintBits = DSR_HINT_WHOLE_SOME | DSR_HINT_WHOLE_ALL | DSR_HINT_VERIFY_FAST | DSR_HINT_TOPK_ALL;
 
 static bool dtype_ok(int32_t d) { return d == DSR_BF16 || d == DSR_F32 || d == DSR_F64; }
@@ -1162,7 +1182,14 @@ static int32_t sample_rows(const dsr_sample_args_t* args, const dsr_head_part_t*
     // on the sliced path; 1 row: 68 against 72).  It has no top-k cut, and
     // the general path takes about 1 ms for such rows: batches of top-k rows
     // go to the sliced path (64 rows, top-k 50: 32 us).
-    launch_full(0u);
+    // Batches of several rounds with greedy rows among them (WHOLE_SOME): see greedy_row.
+    if (a.rows > kFullRows && a.pen_off && (a.hints & DSR_HINT_WHOLE_SOME) && !(a.hints & DSR_HINT_WHOLE_ALL)) {
+      if (a.rng_state) hipLaunchKernelGGL(k_greedy_bf16<true>, dim3((unsigned)a.rows), dim3(kThreads), 0, s, a);
+      else hipLaunchKernelGGL(k_greedy_bf16<false>, dim3((unsigned)a.rows), dim3(kThreads), 0, s, a);
+      launch_full(kModeGreedyDone);
+    } else {
+      launch_full(0u);
+    }
   } else if (f32_path_eligible(a) && !(wide && !parts && a.vocab >= kWideTopkVocab && a.rows * WideLayout(a.vocab).nS <= kWideTopkSlices)) {
     if (a.out_probs_f32 || a.out_probs_f64) {
       const int64_t chunks = (a.vocab + kZeroChunk - 1) / kZeroChunk;
