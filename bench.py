@@ -53,22 +53,22 @@ WORKLOADS = {
     "c3f32": ("sampled rows/sec at B=256×V=129,280 fp32; % of HBM roofline", "rows/s", 5,
               "k_sample_f32"),
     "c1": ("sampled rows/sec at B=1×V=129,280 fp32 with fp32 probabilities out", "rows/s", 1000,
-           "k_zero_probs + k_sample_f32"),
+           "k_wide_scan + k_wide_topk"),
     "c2": ("sampled rows/sec at B=64×V=129,280 bf16 with 4,096-token histories", "rows/s", 20,
            "k_sample_bf16_full"),
     "c4": ("verify-rows/sec at B=32 requests × K=4 drafts × V=129,280 fp32", "verify-rows/s", 60,
            "k_verify_stats + k_verify_chain + k_verify_draw + k_verify_finish"),
     "c5": ("sampled rows/sec at B=1024×V=129,280 bf16, mixed greedy, 16,384-token histories", "rows/s", 2,
-           "k_sample_bf16_full"),
+           "k_greedy_bf16 + k_sample_bf16_full"),
     "hist": ("history rows/sec: 1,024 rows x 16,384 token ids -> sparse count tables over V=129,280", "rows/s", 10,
              "k_history_append (count) + k_history_offsets + k_history_append (write)"),
     "whole": ("sampled rows/sec at B=256×V=129,280 bf16 with no top-k (default / top-p / min-p policies)", "rows/s",
               5, "k_sample_bf16_full"),
     "step": ("drop-in speculative steps/sec: propose 5 rows on the device, verify against 6 fp32 rows, digest",
-             "steps/s", 30, "k_zero_probs + k_sample_f32 (each proposal; the six targets in one launch) + "
+             "steps/s", 30, "k_wide_scan + k_wide_topk (each proposal; the six targets in one launch) + "
              "k_rows_finite + k_vprobs_stats + k_vprobs_chain + k_vprobs_draw + k_vprobs_finish"),
     "seed": ("drop-in TerminalSampler.begin_seed calls/sec (1 fp32 row, V=129,280, dense counts)", "calls/s",
-             300, "k_rows_finite + k_zero_probs + k_sample_f32 (a policy without penalties carries no history "
+             300, "k_rows_finite + k_wide_scan + k_wide_topk (a policy without penalties carries no history "
              "table)"),
     "head": ("verify-rows/sec with the vocabulary projection: B=32 requests × K=4 drafts, 160 target rows × "
              "dim 5,120 → V=129,280 fp32 logits", "verify-rows/s", 30,
@@ -77,7 +77,7 @@ WORKLOADS = {
               "50 sampled from the projection's per-tile records", "rows/s", 32,
               "k_vocab_head + k_sample_f32 (from the records)"),
     "propose": ("drop-in 5-row draft proposal steps/sec at V=129,280 fp32, one host synchronisation per step",
-                "chains/s", 100, "k_zero_probs + k_sample_f32 (5x; a policy without penalties carries no "
+                "chains/s", 100, "k_wide_scan + k_wide_topk (5x; a policy without penalties carries no "
                 "history table)"),
 }
 
