@@ -612,6 +612,7 @@ __global__ __launch_bounds__(kWideThreads) void k_wide_scan(Src src, int nS, int
     if (c) kmin = min(kmin, f32_key(__float_as_uint(mn), true));
   }
   if (r.kept_bits && whole) {  // whole rows keep every finite token
+    if (!touched) lds_barrier();  // every word is clear (uniform; touched rows have passed theirs)
     constexpr int W = DT == DSR_BF16 ? 8 : 4;
 #pragma unroll
     for (int q = 0; q < kWidePer / W; ++q) {
