@@ -865,15 +865,18 @@ __device__ __forceinline__ WideBracket wide_bracket(const WideLayout& L, char* w
   const int b0 = kWideBlocks - 1 - 2 * t;
   double x0 = 0.0, x1 = 0.0;
   {
-    // Slices past the row's read its last one again and scale it by 0 (a
-    // branch would make each load wait for the one before).
+    // Slices past the row's read its last one again (a branch would make each
+    // load wait for the one before).  Theirs count nothing, nor do those of a
+    // slice without a finite token, which k_wide_scan leaves unwritten: a
+    // factor of 0 is selected on, for what lies there may be a NaN.
     float2 q[kWideMaxSlices];
 #pragma unroll
     for (int s = 0; s < kWideMaxSlices; ++s) q[s] = *(const float2*)(h + min(s, L.nS - 1) * kWideBlocks + b0 - 1);
 #pragma unroll
     for (int s = 0; s < kWideMaxSlices; ++s) {
-      x0 += sh.scale[s] * (double)q[s].y;
-      x1 += sh.scale[s] * (double)q[s].x;
+      const double f = sh.scale[s];
+      x0 += f != 0.0 ? f * (double)q[s].y : 0.0;
+      x1 += f != 0.0 ? f * (double)q[s].x : 0.0;
     }
   }
   const double incl = wave_scan_dpp(x0 + x1);
