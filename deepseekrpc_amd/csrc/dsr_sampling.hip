@@ -274,11 +274,12 @@ __global__ __launch_bounds__(kThreads, 8) void k_greedy_bf16(dsr_sample_args_t a
 }
 
 // Sliced path, step three (dsr_wide.h): one workgroup finishes a row from
-// its slices' records, or redoes it on the general path.  Two kernels, each
-// leaving the other's rows untouched (the hints say which are needed):
-// k_wide_topk takes top-k rows and, `others`, greedy rows and rows outside
-// the path's limits; k_wide_draw takes whole rows and always the greedy and
-// outside ones.  `mark` is the path flag of the rows decided here.
+// its slices' records, or redoes it on the general path.  Two kernels (the
+// hints say which are needed): k_wide_topk takes top-k rows and, `others`, all
+// the rest too (whole ones on the general path); k_wide_draw takes all but the
+// top-k rows and, `others`, those too (on the general path).  So every row is
+// decided whatever the hints said of it.  `mark` is the path flag of the rows
+// decided here.
 template <class Src>
 __device__ __forceinline__ void wide_greedy(const Src& src, int64_t row, const RowSpec& r, const WideRow& w, bool draws,
                                             unsigned mark) {
@@ -343,7 +344,7 @@ __global__ __launch_bounds__(kThreads) void k_wide_topk(Src src, int others, uns
 }
 
 template <class Src, int DT, bool RNG>
-__global__ __launch_bounds__(kThreads) void k_wide_draw(Src src, unsigned mark) {
+__global__ __launch_bounds__(kThreads) void k_wide_draw(Src src, int others, unsigned mark) {
   __shared__ WideDrawShared sh;
   const int64_t row = blockIdx.x;
   if (!src.takes(row)) return;
@@ -352,10 +353,12 @@ __global__ __launch_bounds__(kThreads) void k_wide_draw(Src src, unsigned mark) 
   char* ws = src.ws(row);
   const WideLayout L(r.V);
   const WideKind kind = wide_kind(r, L);
-  if (kind == kWideTopK) return;
+  if (kind == kWideTopK && !others) return;
   const int tid = threadIdx.x;
   int why = 0;
-  if (kind == kWideNone) {
+  if (kind == kWideTopK) {
+    why = kHandTopK;
+  } else if (kind == kWideNone) {
     why = wide_outside(r);
   } else {
     const WideRow w = *L.row(ws);
@@ -1056,14 +1059,15 @@ template <class Src, int DT, bool RNG>
 static void wide_launch(const Src& src, int64_t rows, uint32_t hints, bool probs, unsigned mark, hipStream_t s) {
   const int nS = WideLayout(src.a.vocab).nS;
   const dim3 slices((unsigned)(rows * nS)), whole((unsigned)rows);
-  const bool topk_only = hints & DSR_HINT_TOPK_ALL, whole_only = hints & DSR_HINT_WHOLE_ALL;
+  // Both at once contradict each other: the top-k launches decide every row.
+  const bool topk_only = hints & DSR_HINT_TOPK_ALL, whole_only = !topk_only && (hints & DSR_HINT_WHOLE_ALL);
   const int later = probs && !topk_only;
   if (topk_only) hipLaunchKernelGGL((k_wide_scan<Src, DT, false>), slices, dim3(kWideThreads), 0, s, src, nS, later);
   else hipLaunchKernelGGL((k_wide_scan<Src, DT, true>), slices, dim3(kWideThreads), 0, s, src, nS, later);
   if (!topk_only) {
     hipLaunchKernelGGL((k_wide_bracket<Src>), whole, dim3(kBracketThreads), 0, s, src);
     hipLaunchKernelGGL((k_wide_collect<Src, DT>), slices, dim3(kWideThreads), 0, s, src, nS);
-    hipLaunchKernelGGL((k_wide_draw<Src, DT, RNG>), whole, dim3(kThreads), 0, s, src, mark);
+    hipLaunchKernelGGL((k_wide_draw<Src, DT, RNG>), whole, dim3(kThreads), 0, s, src, whole_only ? 1 : 0, mark);
   }
   if (!whole_only)
     hipLaunchKernelGGL((k_wide_topk<Src, DT, RNG>), whole, dim3(kThreads), 0, s, src, topk_only ? 1 : 0, mark);
