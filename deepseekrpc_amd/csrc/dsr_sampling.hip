@@ -321,7 +321,7 @@ __global__ __launch_bounds__(kThreads) void k_wide_topk(Src src, int others, uns
   int st = -1;
   if (kind == kWideTopK || kind == kWideGreedy) {
     double f;
-    const WideRow w = wide_row_of<false>(L, ws, r, nullptr, f);
+    const WideRow w = wide_row_of<false>(L, ws, r, f);
     if (w.bad) {
       why = kHandInvalid;
     } else if (kind == kWideGreedy) {
@@ -373,21 +373,20 @@ __global__ __launch_bounds__(kThreads) void k_wide_draw(Src src, int others, uns
       // overflow on them), stay with the general path.
       why = kHandCapacity;
     } else {
-      exp_table_init(sh.etab);
       if (tid == 0) sh.close = 0u;
       lds_barrier();
       unsigned flags = mark;
       double Sk = 0.0, vc = -INFINITY;
       int32_t ic = INT32_MAX;
       long long npos = 0;
-      const WideKeep every{w.M, r.pol.temperature, -INFINITY, r.pol.min_p, INT32_MAX, sh.etab};
+      const WideKeep every{w.M, r.pol.temperature, 1.0 / r.pol.temperature, -INFINITY, r.pol.min_p, INT32_MAX};
       why = wide_whole(r, L, ws, w, sh, every, vc, ic, Sk, npos, flags);
       if (why == 0) {
         int st = Sk > 0.0 ? DSR_OK : DSR_E_NO_MASS;
         int64_t token = -1;
         int used = 0;
         if (st == DSR_OK && has_draws<RNG>(a)) {
-          const WideKeep K{w.M, r.pol.temperature, vc, r.pol.min_p, ic, sh.etab};
+          const WideKeep K{w.M, r.pol.temperature, every.iT, vc, r.pol.min_p, ic};
           if (npos == 1) {  // sampling.py:120-122: the single positive token; no uniform is drawn
             unsigned none = 0u;
             token = wide_walk<DT>(r, L, ws, sh, K, Sk, npos, 0.0, none);

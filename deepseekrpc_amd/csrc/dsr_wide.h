@@ -347,6 +347,21 @@ __device__ __forceinline__ int wide_block_f(float v) {
   return (int)((b >> 22) ^ (((uint32_t)((int32_t)b >> 31) >> 22) | 0x200u));
 }
 
+// a / T, rounded as the IEEE quotient (sampling.py:88 divides), from iT = 1 / T
+// rounded: a product and one correction by its exact remainder (P. W.
+// Markstein, "Computation of elementary functions on the IBM RISC System/6000
+// processor", IBM J. Res. Dev. 34(1), 1990).  Minus infinity, and a product
+// that overflows to it, give a NaN; wide_exp takes that as minus infinity.
+__device__ __forceinline__ double wide_over(double a, double T, double iT) {
+  const double q = a * iT;
+  return fma(fma(-q, T, a), iT, q);
+}
+
+// exp(z), z <= 0 or a NaN (0; it underflows to 0 below -745.14).  The library's
+// exp, as in the general path: with it and the divide above the scan of 32 FP32
+// rows takes 13.5 us, with exp_nonpos and a product by 1 / T 13.3.
+__device__ __forceinline__ double wide_exp(double z) { return exp(fmax(z, -746.0)); }
+
 // ---------------------------------------------------------------------------
 // Rows of dsr_sample_rows.
 
@@ -393,7 +408,6 @@ struct WideScanShared {
   typename std::conditional<WHOLE, WideHist, None>::type hist;
   uint32_t tbits[kWideSlice / 32];                        // touched tokens
   uint32_t kbits[kWideSlice / 32];                        // finite tokens (kept-bit output)
-  double etab[64];
   WideWaveRec wr[kWideWaves];
   double rs[kWideWaves];
   uint32_t rk[kWideWaves];
@@ -433,7 +447,6 @@ __global__ __launch_bounds__(kWideThreads) void k_wide_scan(Src src, int nS, int
     sh.kbits[t] = 0u;
   }
   if (t < kWidePrefix) sh.found[t] = 0;
-  if (whole) exp_table_init(sh.etab);
   if constexpr (WHOLE) {
     if (hist) {
       uint4* z = (uint4*)&sh.hist;
@@ -724,7 +737,7 @@ __global__ __launch_bounds__(kWideThreads) void k_wide_scan(Src src, int nS, int
       double sum = 0.0;
       unsigned long long* h = sh.hist.w[t & (kWideHistCopies - 1)];
       auto add = [&](double x, int block) {  // x = -inf adds 0, to block 1 (which holds no finite value)
-        const double e = exp_nonpos((x - M) * iT, sh.etab);
+        const double e = wide_exp(wide_over(x - M, p.temperature, iT));
         sum += e;
         if (hist) atomicAdd(&h[block], (unsigned long long)__double_as_longlong(__builtin_fma(e, 0x1p36, kWideOne)));
       };
@@ -781,8 +794,7 @@ __global__ __launch_bounds__(kWideThreads) void k_wide_scan(Src src, int nS, int
 // What the slices' records say about a row, in every lane (uniform).  WHOLE:
 // S, and lane l's factor exp((m - M) / T) of slice l.
 template <bool WHOLE>
-__device__ __forceinline__ WideRow wide_row_of(const WideLayout& L, char* ws, const RowSpec& r, const double* etab,
-                                               double& factor) {
+__device__ __forceinline__ WideRow wide_row_of(const WideLayout& L, char* ws, const RowSpec& r, double& factor) {
   const int l = lane_id();
   WideRow o;
   WideRec x;
@@ -812,7 +824,7 @@ __device__ __forceinline__ WideRow wide_row_of(const WideLayout& L, char* ws, co
     o.vmin = lane_value(row_reduce(x.vmin, OpMin()), 0);
     o.npos = (int32_t)lane_value(row_reduce((uint32_t)x.npos, OpSum()), 0);
     o.crowded = (int)__popcll(__ballot((x.flags & kWideCrowded) != 0u));
-    factor = x.m > -(double)INFINITY ? exp_nonpos((x.m - o.M) / r.pol.temperature, etab) : 0.0;
+    factor = x.m > -(double)INFINITY ? wide_exp((x.m - o.M) / r.pol.temperature) : 0.0;
     o.S = lane_value(row_reduce(factor * x.sum, OpSum()), 0);
   }
   return o;
@@ -845,7 +857,6 @@ struct WideBracketShared {
   double blk[kBracketThreads / 64];
   double pre[kWideBlocks];  // mass per block, inclusive from the top
   double scale[kWideMaxSlices];
-  double etab[64];
   int b[2];
 };
 
@@ -937,12 +948,10 @@ __global__ __launch_bounds__(kBracketThreads) void k_wide_bracket(Src src) {
   const WideKind kind = wide_kind(r, L);
   if (kind != kWideWhole && kind != kWideGreedy) return;
   char* ws = src.ws(d);
-  exp_table_init(sh.etab);
-  lds_barrier();
   WideRow w;
   double f = 0.0;
-  if (kind == kWideGreedy) w = wide_row_of<false>(L, ws, r, nullptr, f);
-  else w = wide_row_of<true>(L, ws, r, sh.etab, f);
+  if (kind == kWideGreedy) w = wide_row_of<false>(L, ws, r, f);
+  else w = wide_row_of<true>(L, ws, r, f);
   if (threadIdx.x < kWideMaxSlices) {
     sh.scale[threadIdx.x] = f;
     L.scale(ws)[threadIdx.x] = f;
@@ -977,7 +986,6 @@ __global__ __launch_bounds__(kBracketThreads) void k_wide_bracket(Src src) {
 }
 
 struct WideCollectShared {
-  double etab[64];
   double rs[kWideWaves], rm[kWideWaves];
   uint32_t rn[kWideWaves], rc[kWideWaves];
   uint32_t tbits[kWideSlice / 32];
@@ -1010,15 +1018,14 @@ __global__ __launch_bounds__(kWideThreads) void k_wide_collect(Src src, int nS) 
   float v[kWidePer];
   wide_load<DT>(r, lo, t, v);
   uint32_t ok = wide_allowed<DT>(r, lo, t);
-  exp_table_init(sh.etab);
   if (touched) {
     if (t < kWideSlice / 32) sh.tbits[t] = 0u;
     lds_barrier();
     wide_touched_each<kWideThreads>(r, rc.e0, rc.e1, rc.b0, rc.b1, lo, hi,
                                     [&](int, int32_t id) { atomicOr(&sh.tbits[(id - lo) >> 5], 1u << ((id - lo) & 31)); });
+    lds_barrier();
+    ok &= ~wide_bits<DT>(sh.tbits, t);
   }
-  lds_barrier();  // the exp table, the touched bits
-  if (touched) ok &= ~wide_bits<DT>(sh.tbits, t);
   // The tokens whose masses are summed go to the wave's LDS list (they are few
   // in most rows, so their exps then fill whole waves); the listed ones are
   // only counted.
@@ -1039,7 +1046,7 @@ __global__ __launch_bounds__(kWideThreads) void k_wide_collect(Src src, int nS) 
   double kept = 0.0, mid = 0.0;
   uint32_t npos = 0u, nt = 0u;
   auto add = [&](double x, bool k) {
-    const double e = exp_nonpos((x - M) * iT, sh.etab);
+    const double e = wide_exp(wide_over(x - M, p.temperature, iT));
     kept += k ? e : 0.0;
     npos += k && e > 0.0 ? 1u : 0u;
     mid += k ? 0.0 : e;
@@ -1111,13 +1118,12 @@ __global__ __launch_bounds__(kWideThreads) void k_wide_collect(Src src, int nS) 
 
 // Tokens a finished whole row keeps, and their weights.
 struct WideKeep {
-  double M, T, vc, min_p;
+  double M, T, iT, vc, min_p;
   int32_t ic;
-  const double* etab;
   __device__ __forceinline__ bool in(double v, int32_t id) const { return (bool)((int)(v > vc) | ((int)(v == vc) & (int)(id <= ic))); }
   // exp((v - M) / T), or 0 below min-p.
   __device__ __forceinline__ double mass(double v) const {
-    const double e = exp_nonpos((v - M) / T, etab);
+    const double e = wide_exp(wide_over(v - M, T, iT));
     return e < min_p ? 0.0 : e;
   }
 };
@@ -1147,7 +1153,6 @@ struct WideDrawShared {
     GenShared g;   // the general path, for rows handed over
   };
   BlockScratch b;
-  double etab[64];
   double Ks[kWideMaxSlices];           // kept mass per slice
   double part[2][kWideMaxSlices];
   uint32_t cnt[2][kWideMaxSlices];
@@ -1187,7 +1192,7 @@ __device__ __forceinline__ double wide_minp_mass(const WideLayout& L, char* ws, 
   double s = 0.0;
   uint32_t close = 0u;
   wide_listed(L, ws, wave, n, [&](double v, int32_t, uint32_t) {
-    const double e = exp_nonpos((v - K.M) / K.T, sh.etab);
+    const double e = wide_exp(wide_over(v - K.M, K.T, K.iT));
     if (e > 0.0 && fabs(e - K.min_p) <= K.min_p * 0x1p-48) close = 1u;
     s += e < K.min_p ? 0.0 : e;
   });
@@ -1289,7 +1294,7 @@ __device__ __forceinline__ int wide_cut(const RowSpec& r, const WideLayout& L, c
   const double before = above + block_exclusive_scan_f64(e, bs, ltot);
   const bool keep = t < nl && (before < P || (t == 0 && nab == 0));
   const int q = (int)block_sum_i64(keep ? 1 : 0, bs);
-  const double tol = ((double)(nab + q) + 16.0) * 0x1p-50 * S;
+  const double tol = ((double)(nab + q) + 16.0) * 0x1p-51 * S;
   const bool near = (t < nl && (t == q || (t == q - 1 && nab + q > 1)) && fabs(before - P) <= tol) ||
                     (t == 0 && q == nl && fabs(above + ltot - P) <= tol);
   if (block_or(near ? 1 : 0, bs)) flags |= DSR_FLAG_MARGIN;
@@ -1396,7 +1401,7 @@ __device__ __forceinline__ int64_t wide_walk(const RowSpec& r, const WideLayout&
                                              const WideKeep& K, double Sk, long long npos, double u, unsigned& flags) {
   const int t = threadIdx.x;
   BlockScratch& bs = sh.b;
-  const double thr = u * Sk, tol = ((double)npos + 16.0) * 0x1p-50 * Sk;
+  const double thr = u * Sk, tol = ((double)npos + 16.0) * 0x1p-51 * Sk;
   int s = -1;
   double base = 0.0, run = 0.0;
   for (int q = 0; q < L.nS; ++q) {
@@ -1658,7 +1663,6 @@ __device__ __forceinline__ int wide_candidates(const RowSpec& r, const WideLayou
 template <class Src, int DT>
 __global__ __launch_bounds__(kWideThreads) void k_wide_probs(Src src, int nS) {
   __shared__ uint32_t tbits[kWideSlice / 32];
-  __shared__ double etab[64];
   const int t = threadIdx.x;
   const int64_t d = blockIdx.x / (unsigned)nS;
   const int s = (int)(blockIdx.x % (unsigned)nS);
@@ -1674,7 +1678,6 @@ __global__ __launch_bounds__(kWideThreads) void k_wide_probs(Src src, int nS) {
   float v[kWidePer];
   wide_load<DT>(r, lo, t, v);
   uint32_t ok = wide_allowed<DT>(r, lo, t);
-  exp_table_init(etab);
   const bool touched = wide_touched(r);
   WideRec rc;
   if (touched) {
@@ -1686,8 +1689,7 @@ __global__ __launch_bounds__(kWideThreads) void k_wide_probs(Src src, int nS) {
     __syncthreads();
     ok &= ~wide_bits<DT>(tbits, t);
   }
-  __syncthreads();  // the exp table
-  const WideKeep K{M, r.pol.temperature, dec.vc, r.pol.min_p, dec.ic, etab};
+  const WideKeep K{M, r.pol.temperature, 1.0 / r.pol.temperature, dec.vc, r.pol.min_p, dec.ic};
   auto prob = [&](double x, int32_t id) { return x > -(double)INFINITY && K.in(x, id) ? K.mass(x) / dec.Sk : 0.0; };
   constexpr int W = 4;
 #pragma unroll

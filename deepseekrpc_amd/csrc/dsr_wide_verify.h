@@ -89,7 +89,7 @@ __global__ __launch_bounds__(kThreads) void k_wide_dist(WideVerifyRows src, int 
   unsigned flags = 0;
   if (kind == kWideTopK || kind == kWideGreedy) {
     double f;
-    const WideRow w = wide_row_of<false>(L, ws, r, nullptr, f);
+    const WideRow w = wide_row_of<false>(L, ws, r, f);
     if (!w.bad && kind == kWideGreedy) {
       form = kFormOne;
       st = DSR_OK;
@@ -122,13 +122,12 @@ __global__ __launch_bounds__(kThreads) void k_wide_dist(WideVerifyRows src, int 
   } else if (kind == kWideWhole && whole) {
     const WideRow w = *L.row(ws);
     if (!w.bad) {
-      exp_table_init(sh.w.etab);
       if (tid == 0) sh.w.close = 0u;
       lds_barrier();
       double Sk = 0.0, vc = -INFINITY;
       int32_t ic = INT32_MAX;
       long long npos = 0;
-      const WideKeep every{w.M, r.pol.temperature, -INFINITY, r.pol.min_p, INT32_MAX, sh.w.etab};
+      const WideKeep every{w.M, r.pol.temperature, 1.0 / r.pol.temperature, -INFINITY, r.pol.min_p, INT32_MAX};
       why = wide_whole(r, L, ws, w, sh.w, every, vc, ic, Sk, npos, flags);
       if (why == 0) {
         form = kFormWhole;
@@ -146,16 +145,15 @@ __global__ __launch_bounds__(kThreads) void k_wide_dist(WideVerifyRows src, int 
   }
 }
 
-// A whole row's kept set as its workspace holds it.
-__device__ __forceinline__ WideKeep wide_kept(const RowSpec& r, const WideLayout& L, char* ws, const double* etab, double& iS) {
+// A whole row's kept set as its workspace holds it, and its mass.
+__device__ __forceinline__ WideKeep wide_kept(const RowSpec& r, const WideLayout& L, char* ws, double& S) {
   const WideDec c = *L.dec(ws);
-  iS = 1.0 / c.Sk;
-  return WideKeep{L.row(ws)->M, r.pol.temperature, c.vc, r.pol.min_p, c.ic, etab};
+  S = c.Sk;
+  return WideKeep{L.row(ws)->M, r.pol.temperature, 1.0 / r.pol.temperature, c.vc, r.pol.min_p, c.ic};
 }
 
 // Token x's probability in distribution d, by one wave (every lane gets it).
-__device__ __forceinline__ double wide_prob_at(const dsr_verify_args_t& a, const VerifyLayout& L, int64_t row, int slot, int32_t x,
-                                               const double* etab) {
+__device__ __forceinline__ double wide_prob_at(const dsr_verify_args_t& a, const VerifyLayout& L, int64_t row, int slot, int32_t x) {
   const int32_t* info = L.info + (row * L.slots + slot) * 4;
   char* ws = (char*)(L.W + (row * L.slots + slot) * L.stride);
   if (info[0] != DSR_OK || x < 0 || x >= a.vocab) return 0.0;
@@ -170,8 +168,8 @@ __device__ __forceinline__ double wide_prob_at(const dsr_verify_args_t& a, const
   }
   const RowSpec r = verify_row_spec(a, L, row, slot);
   const WideLayout W(r.V);
-  double iS;
-  const WideKeep k = wide_kept(r, W, ws, etab, iS);
+  double S;
+  const WideKeep k = wide_kept(r, W, ws, S);
   // Its place among the touched values: the history's, the prefix's first, the bias's.
   int64_t at = -1;
   int e0 = 0, e1 = 0;
@@ -186,7 +184,7 @@ __device__ __forceinline__ double wide_prob_at(const dsr_verify_args_t& a, const
   double v = -INFINITY;
   if (at >= 0) v = W.tv(ws)[at];
   else if (allowed_bit(r.allow, x)) v = load_logit(r.logits, r.dtype, x);
-  return v > -(double)INFINITY && k.in(v, x) ? k.mass(v) * iS : 0.0;
+  return v > -(double)INFINITY && k.in(v, x) ? k.mass(v) / S : 0.0;
 }
 
 // The draw over a top-k request's lists: max(p - q, 0) in index order
@@ -219,7 +217,7 @@ __device__ __forceinline__ int wide_list_draw(const WideList* P, const WideList*
   } else {
     if (!(u >= 0.0 && u < 1.0)) return DSR_E_UNIFORM;
     used = 1;
-    const double thr = u * total, tol = ((double)npos + 16.0) * 0x1p-50 * total + 0x1p-46;
+    const double thr = u * total, tol = ((double)npos + 16.0) * 0x1p-51 * total + 0x1p-46;
     pick = block_min_i64(x > 0.0 && before + x > thr ? (long long)t : LLONG_MAX, bs);
     bool margin = pick == LLONG_MAX;  // rounding left no crossing: the last positive token
     if (margin) pick = block_max_i64(x > 0.0 ? (long long)t : -1ll, bs);
@@ -238,19 +236,18 @@ struct WideWeights {
   RowSpec p, q;
   char *wp, *wq;
   WideKeep kp, kq;
-  double ip, iq;
+  double sp, sq;
   bool resid;
   __device__ __forceinline__ double operator()(double vp, double vq, int32_t id) const {
-    const double x = vp > -(double)INFINITY && kp.in(vp, id) ? kp.mass(vp) * ip : 0.0;
+    const double x = vp > -(double)INFINITY && kp.in(vp, id) ? kp.mass(vp) / sp : 0.0;
     if (!resid) return x;
-    const double y = vq > -(double)INFINITY && kq.in(vq, id) ? kq.mass(vq) * iq : 0.0;
+    const double y = vq > -(double)INFINITY && kq.in(vq, id) ? kq.mass(vq) / sq : 0.0;
     return fmax(x - y, 0.0);
   }
 };
 
 // Whether request `row` draws here; sets its weights.
-__device__ __forceinline__ bool wide_pending(const dsr_verify_args_t& a, const VerifyLayout& L, int64_t row, const double* etab,
-                                             WideWeights& w) {
+__device__ __forceinline__ bool wide_pending(const dsr_verify_args_t& a, const VerifyLayout& L, int64_t row, WideWeights& w) {
   const int64_t d0 = row * L.slots;
   if (!wide_request(L, row) || L.info[d0 * 4 + 3] != kFormWhole) return false;
   const Decision& d = L.dec[row];
@@ -260,21 +257,20 @@ __device__ __forceinline__ bool wide_pending(const dsr_verify_args_t& a, const V
   w.resid = d.next == 1;
   w.p = verify_row_spec(a, L, row, j);
   w.wp = (char*)(L.W + (d0 + j) * L.stride);
-  w.kp = wide_kept(w.p, W, w.wp, etab, w.ip);
+  w.kp = wide_kept(w.p, W, w.wp, w.sp);
   w.q = w.p;
   w.wq = w.wp;
   w.kq = w.kp;
-  w.iq = w.ip;
+  w.sq = w.sp;
   if (w.resid) {
     w.q = verify_row_spec(a, L, row, a.K + 1 + j);
     w.wq = (char*)(L.W + (d0 + a.K + 1 + j) * L.stride);
-    w.kq = wide_kept(w.q, W, w.wq, etab, w.iq);
+    w.kq = wide_kept(w.q, W, w.wq, w.sq);
   }
   return true;
 }
 
 struct WideResidualShared {
-  double etab[64];
   double s[kWideWaves];
   uint32_t n[kWideWaves], f[kWideWaves];
   uint32_t tbits[kWideSlice / 32];
@@ -287,14 +283,13 @@ __global__ __launch_bounds__(kWideThreads) void k_wide_residual(dsr_verify_args_
   const int64_t row = blockIdx.x / (unsigned)nS;
   const int s = (int)(blockIdx.x % (unsigned)nS);
   WideWeights w;
-  if (!wide_pending(a, L, row, sh.etab, w)) return;
+  if (!wide_pending(a, L, row, w)) return;
   const WideLayout W(a.vocab);
   const int lo = s * kWideSlice, hi = lo + kWideSlice < (int)a.vocab ? lo + kWideSlice : (int)a.vocab;
   float vp[kWidePer], vq[kWidePer];
   wide_load<DT>(w.p, lo, t, vp);
   wide_load<DT>(w.q, lo, t, vq);
   uint32_t ok = wide_allowed<DT>(w.p, lo, t);
-  exp_table_init(sh.etab);
   const bool touched = wide_touched(w.p);
   WideRec rc;
   if (touched) {
@@ -303,9 +298,9 @@ __global__ __launch_bounds__(kWideThreads) void k_wide_residual(dsr_verify_args_
     lds_barrier();
     wide_touched_each<kWideThreads>(w.p, rc.e0, rc.e1, rc.b0, rc.b1, lo, hi,
                                     [&](int, int32_t id) { atomicOr(&sh.tbits[(id - lo) >> 5], 1u << ((id - lo) & 31)); });
+    lds_barrier();
+    ok &= ~wide_bits<DT>(sh.tbits, t);
   }
-  lds_barrier();  // the exp table, the touched bits
-  if (touched) ok &= ~wide_bits<DT>(sh.tbits, t);
   double sum = 0.0;
   uint32_t npos = 0u, first = (uint32_t)INT32_MAX;
   auto add = [&](double x, double y, int32_t id) {
@@ -350,7 +345,6 @@ __global__ __launch_bounds__(kWideThreads) void k_wide_residual(dsr_verify_args_
 static_assert(kWideMaxSlices <= kDrawSplit && kWideSlice / 32 == kWideThreads, "a part per slice, a word per thread");
 
 struct WideResolveShared {
-  double etab[64];
   BlockScratch b;
   double vals[kWideSlice];                                   // the slice's touched weights
   uint32_t tbits[kWideSlice / 32], fbits[kWideSlice / 32];  // touched; positive ones
@@ -363,9 +357,8 @@ __global__ __launch_bounds__(kThreads) void k_wide_resolve(dsr_verify_args_t a, 
   const int t = threadIdx.x;
   const int64_t row = blockIdx.x;
   WideWeights w;
-  if (!wide_pending(a, L, row, sh.etab, w)) return;
+  if (!wide_pending(a, L, row, w)) return;
   const WideLayout W(a.vocab);
-  exp_table_init(sh.etab);
   Decision d = L.dec[row];
   // Every thread reads the slices' parts: sums in slice order.
   const DrawPart* parts = L.dpart + row * kDrawSplit;
@@ -391,7 +384,7 @@ __global__ __launch_bounds__(kThreads) void k_wide_resolve(dsr_verify_args_t a, 
   }
   if (used) {  // uniform
     // The last slice with mass that starts at or below the crossing.
-    const double thr = u * total, tol = ((double)npos + 16.0) * 0x1p-50 * total + 0x1p-46;
+    const double thr = u * total, tol = ((double)npos + 16.0) * 0x1p-51 * total + 0x1p-46;
     int s = 0;
     double base = 0.0, run = 0.0;
     for (int q = 0; q < W.nS; ++q) {
@@ -408,7 +401,7 @@ __global__ __launch_bounds__(kThreads) void k_wide_resolve(dsr_verify_args_t a, 
       sh.tbits[t] = 0u;
       sh.fbits[t] = 0u;
     }
-    lds_barrier();  // the exp table, the clear bitmaps
+    lds_barrier();  // the clear bitmaps
     if (touched) {
       const WideRec rc = W.rec(w.wp)[s];
       const double *tp = W.tv(w.wp), *tq = W.tv(w.wq);
@@ -479,7 +472,6 @@ __global__ __launch_bounds__(kThreads) void k_wide_resolve(dsr_verify_args_t a, 
 }
 
 struct WideChainShared {
-  double etab[64];
   double prob[2 * DSR_MAX_DRAFTS + 1];
   double qp[kSplitMaxK];
   int32_t qid[kSplitMaxK];
@@ -495,12 +487,10 @@ __device__ __forceinline__ void wide_decide(const dsr_verify_args_t& a, const Ve
   const int K = a.K;
   const int32_t* info = L.info + row * L.slots * 4;
   const bool greedy = a.policy[row].temperature == 0.0;
-  exp_table_init(ws.etab);
-  __syncthreads();
   const int slot = __builtin_amdgcn_readfirstlane(wave_id());
   if (slot < (int)L.slots && slot != K) {
     const int j = slot < K ? slot : slot - K - 1;
-    const double p = wide_prob_at(a, L, row, slot, a.draft_ids[row * K + j], ws.etab);
+    const double p = wide_prob_at(a, L, row, slot, a.draft_ids[row * K + j]);
     if (lane_id() == 0) ws.prob[slot] = p;
   }
   __syncthreads();

@@ -1,0 +1,38 @@
+"""Float64 probabilities of the sliced path carry one exp and one divide each:
+their ratios against the exact exponential of the IEEE quotient (v - M) / T
+(sampling.py:86-106)."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+from deepseekrpc_amd import _native as N
+from deepseekrpc_amd import batch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("T", [0.7, 1.0, 1.3, 7.1])
+def test_masses_are_one_exp_of_the_ieee_quotient(T):
+    rng = np.random.default_rng(int(10 * T))
+    V, B = 8192, 4
+    x = rng.uniform(-690 * T, 0, (B, V)).astype(np.float32)
+    x[:, 17] = 0.0
+    x[1] += np.float32(3.25)
+    pols = [dict(temperature=T), dict(temperature=T), dict(temperature=T, min_p=0.01), dict(temperature=T, top_p=0.999)]
+    res = batch.sample_rows(torch.from_numpy(x).cuda(), pols, probs="f64")
+    torch.cuda.synchronize()
+    assert (res.flags & N.FLAG_SPLIT).all() and (res.status == 0).all()
+    p = res.probs.cpu().numpy()
+    for r in range(B):
+        keep = p[r] > 0
+        z = (x[r].astype(np.float64) - x[r].astype(np.float64).max()) / T
+        exact = np.exp(z.astype(np.longdouble))[keep]
+        got = p[r].astype(np.longdouble)[keep] / np.longdouble(p[r].max())
+        # The library's exp within 3/4 ulp, the two divides half an ulp each: 1.5 + 1 + 1 times 2^-53 if all three
+        # results lay at the low end of their binades, which the maximum's (one a row) and these masses do not.
+        # Measured 2.5; a table-driven exp of 2 ulps gives 3.1 and more.
+        worst = float(np.max(np.abs(got - exact) / exact))
+        print(r, worst / 2.0**-53, flush=True)
+        assert worst <= 3.0 * 2.0**-53, (r, worst / 2.0**-53)
