@@ -1051,6 +1051,7 @@ constexpr int64_t kWideTopkVocab = 32768;
 static bool wide_path_eligible(const dsr_sample_args_t& a) {
   return (a.dtype == DSR_BF16 || a.dtype == DSR_F32) && a.vocab >= kWideMinVocab && a.rows > 0 &&
          (a.hints & (DSR_HINT_WHOLE_SOME | DSR_HINT_WHOLE_ALL | DSR_HINT_TOPK_ALL)) &&
+         ((uintptr_t)a.workspace & 15u) == 0 &&  // its records, keys and block masses are read 16 bytes at a time
          a.rows * (int64_t)WideLayout(a.vocab).nS * kWideThreads < ((int64_t)1 << 32);
 }
 
