@@ -869,6 +869,8 @@ def verify_drafts(target: torch.Tensor, draft: torch.Tensor, draft_ids: torch.Te
         a.bias_off, a.bias_ids, a.bias_val = bias.offsets.data_ptr(), bias.ids.data_ptr(), bias.values.data_ptr()
     if allow_bits is not None:
         _require_cuda(allow_bits, "allow_bits")
+        if allow_bits.element_size() != 4 or allow_bits.numel() != rows * (K + 1) * allow_bits.shape[-1]:
+            raise ValueError("allow_bits must be [rows, K+1, words] 32-bit: one mask per target row")
         a.allow_bits, a.allow_ld = allow_bits.data_ptr(), allow_bits.shape[-1]
     a.hints = _verify_call_hints(getattr(policies, "dsr_policies", None), V,
                                  not _nonempty(history, "ids") and not _nonempty(bias, "ids") and allow_bits is None) \
