@@ -259,6 +259,31 @@ __device__ __forceinline__ uint32_t wide_bits(const uint32_t* bm, int t) {
   return m;
 }
 
+// FP32 bits of the four tokens from i (a multiple of 4) on; those past the row are -inf.
+template <int DT>
+__device__ __forceinline__ void wide_quad(const RowSpec& r, int64_t i, uint32_t w[4]) {
+  if (i + 4 <= r.V) {
+    if constexpr (DT == DSR_BF16) {
+      struct __attribute__((packed, aligned(2))) Q { uint32_t w[2]; };
+      const Q x = *(const Q*)((const uint16_t*)r.logits + i);
+      w[0] = x.w[0] << 16;
+      w[1] = x.w[0] & 0xFFFF0000u;
+      w[2] = x.w[1] << 16;
+      w[3] = x.w[1] & 0xFFFF0000u;
+    } else {
+      const WideQ4 x = *(const WideQ4*)((const float*)r.logits + i);
+      w[0] = x.w[0]; w[1] = x.w[1]; w[2] = x.w[2]; w[3] = x.w[3];
+    }
+  } else {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const bool in = i + e < r.V;
+      if constexpr (DT == DSR_BF16) w[e] = in ? (uint32_t)((const uint16_t*)r.logits)[i + e] << 16 : 0xFF800000u;
+      else w[e] = in ? ((const uint32_t*)r.logits)[i + e] : 0xFF800000u;
+    }
+  }
+}
+
 // ---------------------------------------------------------------------------
 // Touched tokens.
 
@@ -319,6 +344,18 @@ __device__ __forceinline__ void wide_touched_each(const RowSpec& r, int e0, int 
     if (id >= lo && id < hi) f((int)r.pen_n + (int)threadIdx.x, id);
   }
   for (int b = b0 + (int)threadIdx.x; b < b1; b += STRIDE) f((int)r.pen_n + kWidePrefix + b, r.bias_ids[b]);
+}
+
+// The same by one wave.
+template <class F>
+__device__ __forceinline__ void wide_touched_wave(const RowSpec& r, const WideRec& rc, int64_t lo, int64_t hi, F f) {
+  const int l = lane_id();
+  for (int e = rc.e0 + l; e < rc.e1; e += 64) f(e, r.pen_ids[e]);
+  if (l < r.prefix_n) {
+    const int32_t id = r.prefix[l];
+    if (id >= lo && id < hi) f((int)r.pen_n + l, id);
+  }
+  for (int b = rc.b0 + l; b < rc.b1; b += 64) f((int)r.pen_n + kWidePrefix + b, r.bias_ids[b]);
 }
 
 // Order key of the largest float not above v (finite v), as f32_key orders floats.
@@ -1136,6 +1173,8 @@ struct WideItem {  // a token of the boundary bin
 
 struct WideCut {
   unsigned long long bm[kWideBlocks];  // fixed-point mass per sub-bin of the listed blocks
+  uint32_t bn[kWideBlocks];            // and the tokens in it
+  uint32_t tb[kWideMaxSlices][kWideSlice / 32];  // touched tokens, per slice (a row read again)
   WideItem list[kWideFine];
   double sv[kWideFine], sm[kWideFine];  // the list in rank order, and its masses
   int32_t si[kWideFine];
@@ -1156,42 +1195,89 @@ struct WideDrawShared {
   double Ks[kWideMaxSlices];           // kept mass per slice
   double part[2][kWideMaxSlices];
   uint32_t cnt[2][kWideMaxSlices];
+  long long run;
   int nlist, bin, tok, margin;
   uint32_t close;
 };
 
-// Calls f(value, id, key) for the listed tokens of slice `wave` (lane-strided,
-// a fixed order; eight loads in flight).
-template <class F>
-__device__ __forceinline__ void wide_listed(const WideLayout& L, char* ws, int wave, int n, F f) {
-  const int w = wave < L.nS ? wave : 0;  // n is 0 past the row's slices
-  const double* cv = L.cand_v(ws, w);
-  const int32_t* ci = L.cand_i(ws, w);
-  constexpr int U = 8;
-  for (int i0 = lane_id(); i0 < n; i0 += 64 * U) {
-    double v[U];
-    int32_t id[U];
+// Where a row's listed tokens are: in the lists of its slices, n in this
+// wave's, or, OVER, in the row itself.
+struct WideItems {
+  int n;
+  WideBracket B;
+};
+
+// Calls f(value, id, key) for the listed tokens of slice `wave` (each by one
+// lane, in a fixed order; eight list entries or four quads of the row in flight).
+template <int DT, bool OVER, class F>
+__device__ __forceinline__ void wide_listed(const RowSpec& r, const WideLayout& L, char* ws, int wave, const WideItems& it,
+                                            const WideCut& c, F f) {
+  if constexpr (!OVER) {
+    const int n = it.n, w = wave < L.nS ? wave : 0;  // n is 0 past the row's slices
+    const double* cv = L.cand_v(ws, w);
+    const int32_t* ci = L.cand_i(ws, w);
+    constexpr int U = 8;
+    for (int i0 = lane_id(); i0 < n; i0 += 64 * U) {
+      double v[U];
+      int32_t id[U];
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int i = min(i0 + 64 * u, n - 1);  // unbranched loads
-      v[u] = cv[i];
-      id[u] = ci[i];
+      for (int u = 0; u < U; ++u) {
+        const int i = min(i0 + 64 * u, n - 1);  // unbranched loads
+        v[u] = cv[i];
+        id[u] = ci[i];
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        if (i0 + 64 * u < n) f(v[u], id[u], wide_floor_key(v[u]));  // an untouched value is a float: its own key
     }
+  } else if (wave < L.nS) {
+    const int64_t lo = (int64_t)wave * kWideSlice, hi = lo + kWideSlice < r.V ? lo + kWideSlice : r.V;
+    const bool touched = wide_touched(r);
+    constexpr int U = 4;
+#pragma unroll 1
+    for (int64_t i0 = lo + 4 * lane_id(); i0 < hi; i0 += 256 * U) {
+      uint32_t w[U][4], ok[U];
 #pragma unroll
-    for (int u = 0; u < U; ++u)
-      if (i0 + 64 * u < n) f(v[u], id[u], wide_floor_key(v[u]));  // an untouched value is a float: its own key
+      for (int u = 0; u < U; ++u) {
+        const int64_t i = i0 + 256 * u;
+        wide_quad<DT>(r, i, w[u]);  // slices start at multiples of 1,024: past this one lies the row's end
+        ok[u] = i < hi ? (r.allow ? r.allow[i >> 5] >> (i & 31) : 0xFu) : 0u;
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int64_t i = i0 + 256 * u;
+        if (touched && i < hi) ok[u] &= ~(c.tb[wave][(i - lo) >> 5] >> (i & 31));
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float v = __uint_as_float(w[u][e]);
+          const int b = wide_block_f(v);
+          if (((ok[u] >> e) & 1u) && v > -INFINITY && !it.B.kept(b) && it.B.listed(b))
+            f((double)v, (int32_t)(i + e), f32_key(w[u][e], true));
+        }
+      }
+    }
+    if (touched) {
+      const double* tv = L.tv(ws);
+      wide_touched_wave(r, L.rec(ws)[wave], lo, hi, [&](int at, int32_t id) {
+        const double x = tv[at];
+        const uint32_t key = wide_floor_key(x);
+        const int b = wide_block(key);
+        if (x > -(double)INFINITY && !it.B.kept(b) && it.B.listed(b)) f(x, id, key);
+      });
+    }
   }
 }
 
 // The min-p mass of a row (sampling.py:94-96: kept when r >= min_p * max(r)):
 // the mass above the listed blocks and between them, and the listed tokens
 // themselves.
-__device__ __forceinline__ double wide_minp_mass(const WideLayout& L, char* ws, int n, const WideSum& mine, WideDrawShared& sh,
-                                                 const WideKeep& K, unsigned& flags) {
+template <int DT, bool OVER>
+__device__ __forceinline__ double wide_minp_mass(const RowSpec& r, const WideLayout& L, char* ws, const WideItems& it,
+                                                 const WideSum& mine, WideDrawShared& sh, const WideKeep& K, unsigned& flags) {
   const int wave = __builtin_amdgcn_readfirstlane(wave_id());
   double s = 0.0;
   uint32_t close = 0u;
-  wide_listed(L, ws, wave, n, [&](double v, int32_t, uint32_t) {
+  wide_listed<DT, OVER>(r, L, ws, wave, it, sh.c, [&](double v, int32_t, uint32_t) {
     const double e = wide_exp(wide_over(v - K.M, K.T, K.iT));
     if (e > 0.0 && fabs(e - K.min_p) <= K.min_p * 0x1p-48) close = 1u;
     s += e < K.min_p ? 0.0 : e;
@@ -1208,53 +1294,70 @@ __device__ __forceinline__ double wide_minp_mass(const WideLayout& L, char* ws, 
 
 // The top-p cut of a whole row (sampling.py:97-102): the last kept token, by
 // value and index, into K, and the kept listed mass and positive count of
-// each slice into `s`, `c` of its wave.  `n` tokens are listed for this
-// wave's slice; `base` is the mass certainly kept (nbase positive tokens), S
-// the row's.  Returns 0 or the reason the general path must decide the row.
-__device__ __forceinline__ int wide_cut(const RowSpec& r, const WideLayout& L, char* ws, const WideRow& row, int n, double base,
-                                        long long nbase, double S, WideDrawShared& sh, const WideKeep& K, double& vc, int32_t& ic, double& s,
-                                        uint32_t& c, unsigned& flags) {
+// each slice into `s`, `c` of its wave.  `base` is the mass certainly kept
+// (nbase positive tokens), S the row's.  Returns 0 or the reason the general
+// path must decide the row.
+template <int DT, bool OVER>
+__device__ __forceinline__ int wide_cut(const RowSpec& r, const WideLayout& L, char* ws, const WideRow& row, const WideItems& it,
+                                        double base, long long nbase, double S, WideDrawShared& sh, const WideKeep& K, double& vc,
+                                        int32_t& ic, double& s, uint32_t& c, unsigned& flags) {
   const int t = threadIdx.x, lane = lane_id();
   const int wave = __builtin_amdgcn_readfirstlane(wave_id());
   const int nS = L.nS;
   BlockScratch& bs = sh.b;
   // Fixed-point mass per sub-bin of the order keys of the listed blocks, then
-  // the bin that holds top_p * S.
+  // the bin that holds top_p * S.  OVER: a bin of more tokens than the list
+  // below takes is cut into 1,024 in turn, down to single keys.
   const int blo = row.plo < row.mlo ? row.plo : row.mlo;
-  const uint32_t klo = (uint32_t)blo << 22;
-  const int shift = 12 + max(0, 32 - (int)__clz(max(0, row.hi - blo)));  // (hi - lo + 1) << 22 >> shift <= 1,024
-  sh.c.bm[t] = 0ull;
-  if (t == 0) {
-    sh.bin = -1;
-    sh.nlist = 0;
-  }
-  lds_barrier();
-  wide_listed(L, ws, wave, n, [&](double v, int32_t, uint32_t key) {
-    const double e = K.mass(v);
-    if (e > 0.0) atomicAdd(&sh.c.bm[(key - klo) >> shift], (unsigned long long)(e * 0x1p45));
-  });
-  lds_barrier();
+  uint32_t klo = (uint32_t)blo << 22;
+  int shift = 12 + max(0, 32 - (int)__clz(max(0, row.hi - blo)));  // (hi - lo + 1) << 22 >> shift <= 1,024
   const double P = r.pol.top_p * S;
-  const long long b45 = (long long)(base * 0x1p45);
+  long long run0 = (long long)(base * 0x1p45);  // mass above the bins
   long long tgt = (long long)(P * 0x1p45);
   if (tgt < 1) tgt = 1;
-  const long long mass = (long long)sh.c.bm[kWideBlocks - 1 - t];
-  long long tot;
-  const long long run = b45 + block_exclusive_scan_i64(mass, bs, tot);
-  if (run < tgt && tgt <= run + mass) sh.bin = kWideBlocks - 1 - t;
-  lds_barrier();
+  if (t == 0) sh.nlist = 0;
+  int bin;
+  for (;;) {  // uniform; at most four rounds
+    sh.c.bm[t] = 0ull;
+    if (OVER) sh.c.bn[t] = 0u;
+    if (t == 0) sh.bin = -1;
+    lds_barrier();
+    wide_listed<DT, OVER>(r, L, ws, wave, it, sh.c, [&](double v, int32_t, uint32_t key) {
+      const uint32_t b = (key - klo) >> shift;
+      if (OVER && (key < klo || b >= (uint32_t)kWideBlocks)) return;
+      const double e = K.mass(v);
+      if (OVER) atomicAdd(&sh.c.bn[b], 1u);
+      if (e > 0.0) atomicAdd(&sh.c.bm[b], (unsigned long long)(e * 0x1p45));
+    });
+    lds_barrier();
+    const long long mass = (long long)sh.c.bm[kWideBlocks - 1 - t];
+    long long tot;
+    const long long run = run0 + block_exclusive_scan_i64(mass, bs, tot);
+    if (run < tgt && tgt <= run + mass) {
+      sh.bin = kWideBlocks - 1 - t;
+      sh.run = run;
+    }
+    lds_barrier();
+    bin = sh.bin;
+    if (!OVER || bin < 0 || shift == 0 || sh.c.bn[bin] <= (uint32_t)kWideFine) break;
+    run0 = sh.run;
+    klo += (uint32_t)bin << shift;
+    shift = max(0, shift - 10);
+    lds_barrier();  // every thread has read the bin
+  }
   // A row that cannot be decided still takes every step below, with an empty list.
-  const int bin = sh.bin;
   int why = bin < 0 ? kHandCapacity : 0;  // rounding put the boundary outside the listed tokens
   // The bin's tokens, and the mass and number of listed tokens above it.
+  const uint32_t kbin = klo + ((uint32_t)max(bin, 0) << shift);
   s = 0.0;
   c = 0u;
-  wide_listed(L, ws, wave, n, [&](double v, int32_t id, uint32_t key) {
-    const int b = (int)((key - klo) >> shift);
-    const double e = K.mass(v);
-    s += b > bin ? e : 0.0;
-    c += b > bin && e > 0.0 ? 1u : 0u;
-    if (b == bin) {
+  wide_listed<DT, OVER>(r, L, ws, wave, it, sh.c, [&](double v, int32_t id, uint32_t key) {
+    if (key < kbin) return;
+    if ((key - kbin) >> shift) {
+      const double e = K.mass(v);
+      s += e;
+      c += e > 0.0 ? 1u : 0u;
+    } else {
       const int at = atomicAdd(&sh.nlist, 1);
       if (at < kWideFine) sh.c.list[at] = WideItem{v, id, 0};
     }
@@ -1298,7 +1401,7 @@ __device__ __forceinline__ int wide_cut(const RowSpec& r, const WideLayout& L, c
   const bool near = (t < nl && (t == q || (t == q - 1 && nab + q > 1)) && fabs(before - P) <= tol) ||
                     (t == 0 && q == nl && fabs(above + ltot - P) <= tol);
   if (block_or(near ? 1 : 0, bs)) flags |= DSR_FLAG_MARGIN;
-  const double vk = sh.c.sv[q > 0 ? q - 1 : 0], vr = sh.c.sv[q < nl ? q : nl - 1];  // last kept, first removed
+  const double vk = sh.c.sv[q > 0 ? q - 1 : 0], vr = sh.c.sv[q < nl ? q : max(nl - 1, 0)];  // last kept, first removed
   vc = vk;
   ic = q > 0 ? sh.c.si[q - 1] : -1;
   // Values on the two sides of the cut must stay apart after (v - M) / T, or
@@ -1313,7 +1416,7 @@ __device__ __forceinline__ int wide_cut(const RowSpec& r, const WideLayout& L, c
       if (v < vr) lower = fmax(lower, v);
       if (v > vk) upper = fmin(upper, v);
     };
-    wide_listed(L, ws, wave, n, [&](double v, int32_t, uint32_t) { side(v); });
+    wide_listed<DT, OVER>(r, L, ws, wave, it, sh.c, [&](double v, int32_t, uint32_t) { side(v); });
     const double* tv = L.tv(ws);
     for (int i = t; i < (int)r.pen_n; i += kThreads) side(tv[i]);
     if (t < r.prefix_n) side(tv[r.pen_n + t]);
@@ -1341,11 +1444,12 @@ __device__ __forceinline__ int wide_cut(const RowSpec& r, const WideLayout& L, c
 
 // A whole row: the kept set (K), the kept mass per slice (sh.Ks) and in all
 // (Sk), and its positive tokens.  Returns 0 or the reason the general path
-// must decide the row.  Every thread of the 1,024 calls; wave w works on
-// slice w.
-__device__ __forceinline__ int wide_whole(const RowSpec& r, const WideLayout& L, char* ws, const WideRow& row,
-                                          WideDrawShared& sh, const WideKeep& K, double& vc, int32_t& ic, double& Sk, long long& npos,
-                                          unsigned& flags) {
+// must decide the row, kHandCapacity also when the slices' lists cannot.
+// Every thread of the 1,024 calls; wave w works on slice w.
+template <int DT, bool OVER>
+__device__ __forceinline__ int wide_whole_from(const RowSpec& r, const WideLayout& L, char* ws, const WideRow& row,
+                                               WideDrawShared& sh, const WideKeep& K, double& vc, int32_t& ic, double& Sk,
+                                               long long& npos, unsigned& flags) {
   const int lane = lane_id();
   const int wave = __builtin_amdgcn_readfirstlane(wave_id());
   const dsr_policy_t& p = r.pol;
@@ -1358,18 +1462,27 @@ __device__ __forceinline__ int wide_whole(const RowSpec& r, const WideLayout& L,
     mine.mid = lane_value(all.mid, wave);
     mine.ncand = (int32_t)lane_value((uint32_t)all.ncand, wave);
   }
-  const int n = __builtin_amdgcn_readfirstlane(mine.ncand);
-  int why = __ballot(all.ncand > L.cand_cap()) ? kHandCapacity : 0;  // uniform over the workgroup
+  const WideItems it{__builtin_amdgcn_readfirstlane(mine.ncand), WideBracket{row.hi, row.plo, row.phi, row.mlo, row.mhi}};
+  if (!OVER && __ballot(all.ncand > L.cand_cap())) return kHandCapacity;  // uniform over the workgroup
   const double base = lane_value(row_reduce(all.kept, OpSum()), 0);  // mass certainly kept, and its positive tokens
   const long long nbase = (long long)lane_value(row_reduce((uint32_t)all.npos, OpSum()), 0);
+  if (OVER && wide_touched(r) && wave < nS) {  // the wave's own slice
+    uint32_t* tb = sh.c.tb[wave];
+    const int64_t lo = (int64_t)wave * kWideSlice, hi = lo + kWideSlice < r.V ? lo + kWideSlice : r.V;
+    for (int i = lane; i < kWideSlice / 32; i += 64) tb[i] = 0u;
+    wave_lds_sync();
+    wide_touched_wave(r, L.rec(ws)[wave], lo, hi, [&](int, int32_t id) { atomicOr(&tb[(id - lo) >> 5], 1u << ((id - lo) & 31)); });
+    wave_lds_sync();
+  }
+  int why = 0;
   double s = 0.0;
   uint32_t c = 0u;
-  if (!nof && why == 0) {
-    const double S = p.min_p != 0.0 ? wide_minp_mass(L, ws, n, mine, sh, K, flags) : row.S;
+  if (!nof) {
+    const double S = p.min_p != 0.0 ? wide_minp_mass<DT, OVER>(r, L, ws, it, mine, sh, K, flags) : row.S;
     if (p.top_p < 1.0) {
-      why = wide_cut(r, L, ws, row, n, base, nbase, S, sh, K, vc, ic, s, c, flags);
+      why = wide_cut<DT, OVER>(r, L, ws, row, it, base, nbase, S, sh, K, vc, ic, s, c, flags);
     } else {  // min-p alone
-      wide_listed(L, ws, wave, n, [&](double v, int32_t, uint32_t) {
+      wide_listed<DT, OVER>(r, L, ws, wave, it, sh.c, [&](double v, int32_t, uint32_t) {
         const double e = K.mass(v);
         s += e;
         c += e > 0.0 ? 1u : 0u;
@@ -1390,6 +1503,28 @@ __device__ __forceinline__ int wide_whole(const RowSpec& r, const WideLayout& L,
   for (int q = 0; q < nS; ++q) {
     Sk += sh.Ks[q];
     npos += sh.cnt[1][q];
+  }
+  return why;
+}
+
+// The same from the slices' lists, and again from the row where they cannot
+// tell: a slice lists more tokens than its list holds, or the cut's sub-bin more
+// than are ranked.  Blocks and sub-bins follow the logit itself, so that takes
+// logits with a common offset (N(0, 1) at +-70 and beyond) or nearly equal
+// ones.  A pass over a row of 129,280 is read at one workgroup's pace; the
+// general path, which such rows would take, needs 22.
+template <int DT>
+__device__ __forceinline__ int wide_whole(const RowSpec& r, const WideLayout& L, char* ws, const WideRow& row,
+                                          WideDrawShared& sh, const WideKeep& K, double& vc, int32_t& ic, double& Sk, long long& npos,
+                                          unsigned& flags) {
+  const unsigned flags0 = flags;
+  int why = wide_whole_from<DT, false>(r, L, ws, row, sh, K, vc, ic, Sk, npos, flags);
+  if (why == kHandCapacity && !wide_nofilter(r.pol)) {  // uniform
+    __syncthreads();  // every thread is done with the first attempt's LDS
+    if (threadIdx.x == 0) sh.close = 0u;
+    lds_barrier();
+    flags = flags0;
+    why = wide_whole_from<DT, true>(r, L, ws, row, sh, K, vc, ic, Sk, npos, flags);
   }
   return why;
 }
@@ -1577,26 +1712,7 @@ __device__ __forceinline__ int wide_candidates(const RowSpec& r, const WideLayou
   auto quad = [&](int item, float v[4]) -> uint32_t {  // bit e: candidate; v: values
     const int64_t i = (int64_t)gl[item >> 2] * kWideGroup + 4 * (item & 3);
     uint32_t w[4];
-    if (i + 4 <= r.V) {
-      if constexpr (DT == DSR_BF16) {
-        struct __attribute__((packed, aligned(2))) Q { uint32_t w[2]; };
-        const Q x = *(const Q*)((const uint16_t*)r.logits + i);
-        w[0] = x.w[0] << 16;
-        w[1] = x.w[0] & 0xFFFF0000u;
-        w[2] = x.w[1] << 16;
-        w[3] = x.w[1] & 0xFFFF0000u;
-      } else {
-        const WideQ4 x = *(const WideQ4*)((const float*)r.logits + i);
-        w[0] = x.w[0]; w[1] = x.w[1]; w[2] = x.w[2]; w[3] = x.w[3];
-      }
-    } else {
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const bool in = i + e < r.V;
-        if constexpr (DT == DSR_BF16) w[e] = in ? (uint32_t)((const uint16_t*)r.logits)[i + e] << 16 : 0xFF800000u;
-        else w[e] = in ? ((const uint32_t*)r.logits)[i + e] : 0xFF800000u;
-      }
-    }
+    wide_quad<DT>(r, i, w);
     uint32_t ok = 0xFu;
     if (i < r.V) {
       if (r.allow) ok &= r.allow[i >> 5] >> (i & 31);

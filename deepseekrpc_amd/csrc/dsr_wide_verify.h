@@ -128,7 +128,7 @@ __global__ __launch_bounds__(kThreads) void k_wide_dist(WideVerifyRows src, int 
       int32_t ic = INT32_MAX;
       long long npos = 0;
       const WideKeep every{w.M, r.pol.temperature, 1.0 / r.pol.temperature, -INFINITY, r.pol.min_p, INT32_MAX};
-      why = wide_whole(r, L, ws, w, sh.w, every, vc, ic, Sk, npos, flags);
+      why = wide_whole<DT>(r, L, ws, w, sh.w, every, vc, ic, Sk, npos, flags);
       if (why == 0) {
         form = kFormWhole;
         st = Sk > 0.0 ? DSR_OK : DSR_E_NO_MASS;
