@@ -1397,6 +1397,9 @@ __device__ __forceinline__ int wide_cut(const RowSpec& r, const WideLayout& L, c
   const double before = above + block_exclusive_scan_f64(e, bs, ltot);
   const bool keep = t < nl && (before < P || (t == 0 && nab == 0));
   const int q = (int)block_sum_i64(keep ? 1 : 0, bs);
+  // The last kept token starts below P and reaches it.  A bin without it: the
+  // fixed-point sums (each mass cut to 2^-45) put the boundary a bin too low.
+  if (!why && (q == 0 || above + ltot < P)) why = kHandCapacity;
   const double tol = ((double)(nab + q) + 16.0) * 0x1p-51 * S;
   const bool near = (t < nl && (t == q || (t == q - 1 && nab + q > 1)) && fabs(before - P) <= tol) ||
                     (t == 0 && q == nl && fabs(above + ltot - P) <= tol);
