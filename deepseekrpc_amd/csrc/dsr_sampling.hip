@@ -309,7 +309,7 @@ __global__ __launch_bounds__(kThreads) void k_wide_topk(Src src, int others, uns
   const RowSpec r = src.spec(row);
   char* ws = src.ws(row);
   const WideLayout L(r.V);
-  const WideKind kind = wide_kind(r, L);
+  const WideKind kind = src.kind(r, L);
   if (kind != kWideTopK && !others) return;
   int why = 0;
   unsigned flags = mark;
@@ -352,7 +352,7 @@ __global__ __launch_bounds__(kThreads) void k_wide_draw(Src src, int others, uns
   const RowSpec r = src.spec(row);
   char* ws = src.ws(row);
   const WideLayout L(r.V);
-  const WideKind kind = wide_kind(r, L);
+  const WideKind kind = src.kind(r, L);
   if (kind == kWideTopK && !others) return;
   const int tid = threadIdx.x;
   int why = 0;
@@ -367,11 +367,6 @@ __global__ __launch_bounds__(kThreads) void k_wide_draw(Src src, int others, uns
     } else if (kind == kWideGreedy) {
       wide_greedy(src, row, r, w, has_draws<RNG>(a), mark);
       return;
-    } else if (wide_nofilter(r.pol) && r.pen_n > 0 && (wide_neutral(r.pol) || 2 * w.crowded > L.nS)) {
-      // No filter: a table that only the count check reads, and rows whose
-      // tokens crowd into one block (the full-vocabulary kernel's key counts
-      // overflow on them), stay with the general path.
-      why = kHandCapacity;
     } else {
       if (tid == 0) sh.close = 0u;
       lds_barrier();

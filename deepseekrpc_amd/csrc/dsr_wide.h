@@ -71,7 +71,6 @@ static_assert((int64_t)kWideMaxSlices * kWideSlice >= DSR_MAX_VOCAB, "the slices
 static_assert(kWideMaxSlices == kWaves, "one wave of the finishing workgroup per slice");
 
 constexpr uint32_t kWideBad = 1u;      // NaN or +inf, or a history / bias entry the general path rejects
-constexpr uint32_t kWideCrowded = 2u;  // a block holds more than half of the slice's tokens
 
 struct WideRec {      // one slice, from k_wide_scan
   double m;           // largest adjusted value (-inf: none)
@@ -89,7 +88,7 @@ static_assert(sizeof(WideRec) == 64, "workspace layout");
 
 struct WideSum {      // one slice, from k_wide_collect
   double kept;        // mass of the tokens certainly kept, relative to the row maximum
-  double mid;         // mass of those min-p keeps and top-p certainly removes
+  double mid;         // with min-p: mass of those it keeps and top-p certainly removes
   int32_t npos;       // positive masses in `kept`
   int32_t ncand;      // listed tokens, or more than the list holds
 };
@@ -101,7 +100,6 @@ struct WideRow {      // one row, from k_wide_bracket
   int32_t first;      // greedy rows: first index holding M
   int32_t npos;       // whole rows with no filter: finite tokens
   int32_t bad;        // invalid: the general path reports it
-  int32_t crowded;    // slices whose tokens crowd into one block
   int32_t hi, plo, phi, mlo, mhi;  // WideBracket
   int32_t pad;
 };
@@ -410,6 +408,11 @@ struct WideSampleRows {
   __device__ __forceinline__ char* ws(int64_t d) const { return (char*)a.workspace + (size_t)d * ws_stride(a.vocab) * sizeof(double); }
   __device__ __forceinline__ RowSpec spec(int64_t d) const { return sample_row_spec(a, d, (double*)ws(d)); }
   __device__ __forceinline__ void onehot(int64_t, int64_t) const {}
+  // Unfiltered rows whose table changes no logit stay on the general path, as before this one.
+  __device__ __forceinline__ WideKind kind(const RowSpec& r, const WideLayout& L) const {
+    const WideKind k = wide_kind(r, L);
+    return k == kWideWhole && r.pen_n > 0 && wide_nofilter(r.pol) && wide_neutral(r.pol) ? kWideNone : k;
+  }
 };
 
 // ---------------------------------------------------------------------------
@@ -424,16 +427,8 @@ struct WideWaveRec {   // one wave's part of a slice
 
 // A token's part of a block's 64-bit word: the bits of the double 2^52 + 2^50
 // + mass * 2^36.  A slice's masses sum below 2^50, so the low 50 bits of a
-// word are their sum and the high 14 its token count times an odd constant.
+// word are their sum (the others mean nothing).
 constexpr double kWideOne = 0x1p52 + 0x1p50;
-constexpr uint32_t kWideOneHigh = (0x433u << 2) | 1u;  // the high 14 bits of kWideOne's
-constexpr uint32_t wide_inverse(uint32_t x) {          // modulo 2^14, by Newton's steps
-  uint32_t y = x;
-  for (int i = 0; i < 4; ++i) y *= 2u - x * y;
-  return y & 0x3FFFu;
-}
-static_assert(((kWideOneHigh * wide_inverse(kWideOneHigh)) & 0x3FFFu) == 1u, "the count can be read back");
-
 struct WideHist {
   // The copies start on different banks.
   unsigned long long w[kWideHistCopies][kWideBlocks + 8];
@@ -447,7 +442,6 @@ struct WideScanShared {
   uint32_t kbits[kWideSlice / 32];                        // finite tokens (kept-bit output)
   WideWaveRec wr[kWideWaves];
   double rs[kWideWaves];
-  uint32_t rk[kWideWaves];
   int found[kWidePrefix];
 };
 
@@ -462,7 +456,7 @@ __global__ __launch_bounds__(kWideThreads) void k_wide_scan(Src src, int nS, int
   if (!src.takes(d)) return;
   const RowSpec r = src.spec(d);
   const WideLayout L(r.V);
-  const WideKind kind = wide_kind(r, L);
+  const WideKind kind = src.kind(r, L);
   if (kind == kWideNone || (!WHOLE && kind == kWideWhole)) return;  // the finishing workgroup's general path
   char* ws = src.ws(d);
   const int lo = s * kWideSlice, hi = lo + kWideSlice < (int)r.V ? lo + kWideSlice : (int)r.V;
@@ -478,7 +472,7 @@ __global__ __launch_bounds__(kWideThreads) void k_wide_scan(Src src, int nS, int
 
   const bool whole = WHOLE && kind == kWideWhole;
   const bool nof = wide_nofilter(p);
-  const bool hist = whole && (!nof || r.pen_n > 0);
+  const bool hist = whole && !nof;  // only filtered rows look for a block
   if (t < kWideSlice / 32) {
     sh.tbits[t] = 0u;
     sh.kbits[t] = 0u;
@@ -802,25 +796,15 @@ __global__ __launch_bounds__(kWideThreads) void k_wide_scan(Src src, int nS, int
       for (int q = 0; q < kWideWaves; ++q) o.sum += sh.rs[q];
       if (hist) {
         float4* ho = (float4*)(L.hist(ws) + s * kWideBlocks) + t;  // blocks 4t .. 4t + 3
-        uint32_t most = 0u;
         float f[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          const int b = 4 * t + i;
           unsigned long long x = 0ull;
 #pragma unroll
-          for (int c = 0; c < kWideHistCopies; ++c) x += sh.hist.w[c][b];
+          for (int c = 0; c < kWideHistCopies; ++c) x += sh.hist.w[c][4 * t + i];
           f[i] = (float)((double)(x & ((1ull << 50) - 1ull)) * 0x1p-36);
-          if (nof && b > 1) most = max(most, ((uint32_t)(x >> 50) * wide_inverse(kWideOneHigh)) & 0x3FFFu);
         }
         *ho = make_float4(f[0], f[1], f[2], f[3]);
-        if (nof) {  // read for these rows alone (uniform)
-          most = wave_reduce_dpp(most, OpMax());
-          if (lane_id() == 0) sh.rk[wave_id()] = most;
-          lds_barrier();
-          for (int q = 0; q < kWideWaves; ++q) most = max(most, sh.rk[q]);
-          if (most > (uint32_t)((hi - lo) / 2)) o.flags |= kWideCrowded;
-        }
       }
     }
   }
@@ -860,7 +844,6 @@ __device__ __forceinline__ WideRow wide_row_of(const WideLayout& L, char* ws, co
   if constexpr (WHOLE) {
     o.vmin = lane_value(row_reduce(x.vmin, OpMin()), 0);
     o.npos = (int32_t)lane_value(row_reduce((uint32_t)x.npos, OpSum()), 0);
-    o.crowded = (int)__popcll(__ballot((x.flags & kWideCrowded) != 0u));
     factor = x.m > -(double)INFINITY ? wide_exp((x.m - o.M) / r.pol.temperature) : 0.0;
     o.S = lane_value(row_reduce(factor * x.sum, OpSum()), 0);
   }
@@ -982,7 +965,7 @@ __global__ __launch_bounds__(kBracketThreads) void k_wide_bracket(Src src) {
   if (!src.takes(d)) return;
   const RowSpec r = src.spec(d);
   const WideLayout L(r.V);
-  const WideKind kind = wide_kind(r, L);
+  const WideKind kind = src.kind(r, L);
   if (kind != kWideWhole && kind != kWideGreedy) return;
   char* ws = src.ws(d);
   WideRow w;
@@ -1013,7 +996,6 @@ __global__ __launch_bounds__(kBracketThreads) void k_wide_bracket(Src src) {
     o->first = w.first;
     o->npos = w.npos;
     o->bad = w.bad;
-    o->crowded = w.crowded;
     o->hi = w.hi;
     o->plo = w.plo;
     o->phi = w.phi;
@@ -1039,7 +1021,7 @@ __global__ __launch_bounds__(kWideThreads) void k_wide_collect(Src src, int nS) 
   if (!src.takes(d)) return;
   const RowSpec r = src.spec(d);
   const WideLayout L(r.V);
-  if (wide_kind(r, L) != kWideWhole) return;
+  if (src.kind(r, L) != kWideWhole) return;
   char* ws = src.ws(d);
   const dsr_policy_t& p = r.pol;
   const WideRow w = *L.row(ws);
@@ -1065,14 +1047,15 @@ __global__ __launch_bounds__(kWideThreads) void k_wide_collect(Src src, int nS) 
   }
   // The tokens whose masses are summed go to the wave's LDS list (they are few
   // in most rows, so their exps then fill whole waves); the listed ones are
-  // only counted.
+  // only counted.  Tokens between the two cuts count for min-p alone.
+  const bool mids = p.min_p != 0.0;
   float* mv = sh.mv[wave];
   uint32_t nm = 0u, sel = 0u;  // nm: uniform
 #pragma unroll
   for (int k = 0; k < kWidePer; ++k) {
     const int b = wide_block_f(v[k]);
     const bool f = ((ok >> k) & 1u) && v[k] > -INFINITY;
-    const bool sum = f && (B.kept(b) || B.middle(b));
+    const bool sum = f && (B.kept(b) || (mids && B.middle(b)));
     if (f && !B.kept(b) && B.listed(b)) sel |= 1u << k;
     const unsigned long long bal = __ballot(sum);
     if (sum) mv[nm + lanes_below(bal)] = v[k];
@@ -1095,7 +1078,7 @@ __global__ __launch_bounds__(kWideThreads) void k_wide_collect(Src src, int nS) 
       if (!(x > -(double)INFINITY)) return;
       const int b = wide_block(wide_floor_key(x));
       const bool k = B.kept(b);
-      if (k || B.middle(b)) add(x, k);
+      if (k || (mids && B.middle(b))) add(x, k);
       if (!k && B.listed(b)) ++nt;
     });
   // Listed tokens go to the slice's list in thread order (a fixed order).
@@ -1788,7 +1771,7 @@ __global__ __launch_bounds__(kWideThreads) void k_wide_probs(Src src, int nS) {
   if (!src.takes(d)) return;
   const RowSpec r = src.spec(d);
   const WideLayout L(r.V);
-  if (wide_kind(r, L) != kWideWhole) return;
+  if (src.kind(r, L) != kWideWhole) return;
   char* ws = src.ws(d);
   const WideDec dec = *L.dec(ws);
   if (dec.done != 0) return;

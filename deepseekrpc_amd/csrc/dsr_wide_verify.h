@@ -53,6 +53,7 @@ struct WideVerifyRows {
   VerifyLayout L;
   dsr_sample_args_t a;  // no draws; the top-k tail's status, per distribution
   __device__ __forceinline__ bool takes(int64_t) const { return true; }
+  __device__ __forceinline__ WideKind kind(const RowSpec& r, const WideLayout& L) const { return wide_kind(r, L); }
   __device__ __forceinline__ char* ws(int64_t d) const { return (char*)(L.W + d * L.stride); }
   __device__ __forceinline__ RowSpec spec(int64_t d) const {
     const uint32_t row = (uint32_t)d / (uint32_t)L.slots;
@@ -82,7 +83,7 @@ __global__ __launch_bounds__(kThreads) void k_wide_dist(WideVerifyRows src, int 
   const RowSpec r = src.spec(d);
   char* ws = src.ws(d);
   const WideLayout L(r.V);
-  const WideKind kind = wide_kind(r, L);
+  const WideKind kind = src.kind(r, L);
   const int tid = threadIdx.x;
   int form = kFormDense, st = -1, why = 0;
   int64_t onehot = -1;

@@ -10,6 +10,7 @@ import pytest
 import torch
 
 from deepseekrpc_amd import _native as N
+from deepseekrpc_amd import workloads
 from test_gpu_wide import PEN, histories, rows_of, sample
 
 pytestmark = pytest.mark.gpu
@@ -51,7 +52,21 @@ def test_bf16_rows(offset):
     rng = np.random.default_rng(4)
     B, V = len(POLICIES), 30000
     x = rows_of(rng, B, V, "normal", torch.bfloat16)
-    from deepseekrpc_amd import workloads
     x = workloads.bf16_round((x + np.float32(offset)).astype(np.float32))
     counts, gens = histories(rng, B, V, 3000)
     sample(x, [dict(p, **PEN) for p in POLICIES], rng.random(B), torch.bfloat16, 1, counts, gens)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_unfiltered_rows_crowded_into_one_block(dtype):
+    """No filter, penalised: the slices' sums decide the row however its tokens lie."""
+    rng = np.random.default_rng(12)
+    V = 20001
+    x = np.concatenate([rows_of(rng, 1, V, "flat", torch.float32) + np.float32(0.003), rows_of(rng, 1, V, "normal", torch.float32),
+                        rows_of(rng, 1, V, "normal", torch.float32) + np.float32(90.0)]).astype(np.float32)
+    if dtype == torch.bfloat16:
+        x = workloads.bf16_round(x)
+    counts, gens = histories(rng, 3, V, 4000)
+    bias = [{5: 0.5, V - 1: -1.0}] * 3  # keeps bf16 rows off the register kernel
+    flags = sample(x, [dict(PEN), dict(PEN, temperature=0.6), dict(PEN)], rng.random(3), dtype, 1, counts, gens, bias)
+    assert (flags & N.FLAG_SPLIT).all(), [hex(int(f)) for f in flags]
