@@ -1607,10 +1607,11 @@ __device__ __forceinline__ int64_t wide_walk(const RowSpec& r, const WideLayout&
 }
 
 // A top-k row's candidates, in index order, in shu.t (cz / cid): every token
-// that can survive top-k.  Returns their number, or -1 with the reason.
+// that can survive top-k.  Returns their number, or -1 where the groups'
+// 16-bit prefixes cannot bound them to the list.
 template <int DT>
-__device__ __forceinline__ int wide_candidates(const RowSpec& r, const WideLayout& L, char* ws, double M, long long k,
-                                               F32Shared& shu, int& why) {
+__device__ __forceinline__ int wide_candidates_prefix(const RowSpec& r, const WideLayout& L, char* ws, double M, long long k,
+                                                      F32Shared& shu) {
   F32Lists& t = shu.t;
   BlockScratch& bs = shu.gen.b;
   const int tid = threadIdx.x, lane = lane_id();
@@ -1664,10 +1665,7 @@ __device__ __forceinline__ int wide_candidates(const RowSpec& r, const WideLayou
     for (int i = 0; i < 8; ++i) f(g[i]);
     if (touched) places([&](int, int32_t, uint32_t x) { f(x); });
   });
-  if (tau16 == 0u) {  // fewer finite groups and touched tokens than k
-    why = kHandCapacity;
-    return -1;
-  }
+  if (tau16 == 0u) return -1;  // fewer finite groups and touched tokens than k
   // The groups to read again (their order does not matter), and the bitmaps.
   uint32_t* gl = &t.hist[0][0];
   constexpr int kCap = kWaves * kF32Bins;
@@ -1689,10 +1687,7 @@ __device__ __forceinline__ int wide_candidates(const RowSpec& r, const WideLayou
     });
   __syncthreads();
   const int n = t.wn[0];
-  if (n > kCap) {
-    why = kHandCapacity;
-    return -1;
-  }
+  if (n > kCap) return -1;
   // Four lanes per group, four tokens each; two passes over the same reads
   // (the second from cache): mark the candidates, then place them.
   auto quad = [&](int item, float v[4]) -> uint32_t {  // bit e: candidate; v: values
@@ -1725,10 +1720,7 @@ __device__ __forceinline__ int wide_candidates(const RowSpec& r, const WideLayou
     const uint4 q = *(const uint4*)&cbm[4 * tid];
     const uint32_t c0 = __popc(q.x), c1 = __popc(q.y), c2 = __popc(q.z), c3 = __popc(q.w);
     const long long ex = block_exclusive_scan_i64((long long)(c0 + c1 + c2 + c3), bs, nc);
-    if (nc > kF32Cap) {
-      why = kHandCapacity;
-      return -1;
-    }
+    if (nc > kF32Cap) return -1;
     uint32_t b = (uint32_t)ex;
     base[4 * tid] = (uint16_t)b;
     base[4 * tid + 1] = (uint16_t)(b += c0);
@@ -1757,6 +1749,165 @@ __device__ __forceinline__ int wide_candidates(const RowSpec& r, const WideLayou
     });
   __syncthreads();
   return (int)nc;
+}
+
+// The same from the tokens themselves: the k-th largest one's whole order key,
+// by four 8-bit radix passes over the row, and every token from it on.  Returns
+// their number, or -1 when a tie group outgrows the list or fewer than k
+// tokens are finite.  Rows that come here: many logits within 2^-7 of the k-th
+// largest (nearly equal ones, or a large common offset), and a top-k near the
+// row's number of 16-token groups.
+template <int DT>
+__device__ __forceinline__ int wide_candidates_exact(const RowSpec& r, const WideLayout& L, char* ws, double M, long long k,
+                                                     F32Shared& shu) {
+  F32Lists& t = shu.t;
+  BlockScratch& bs = shu.gen.b;
+  const int tid = threadIdx.x, lane = lane_id();
+  const int wave = __builtin_amdgcn_readfirstlane(wave_id());
+  uint32_t* tbm = (uint32_t*)t.sp;   // touched tokens
+  uint32_t* cbm = (uint32_t*)t.pos;  // candidates
+  uint16_t* base = (uint16_t*)t.kz;  // candidates below each word
+  const double* tv = L.tv(ws);
+  const bool touched = wide_touched(r);
+  auto places = [&](auto f) {  // place and id
+    for (int e = tid; e < (int)r.pen_n; e += kThreads) f(e, r.pen_ids[e]);
+    if (tid < r.prefix_n) f((int)r.pen_n + tid, r.prefix[tid]);
+    for (int b = tid; b < (int)r.bias_n; b += kThreads) f((int)r.pen_n + kWidePrefix + b, r.bias_ids[b]);
+  };
+  __syncthreads();  // every thread is done with the first attempt's lists
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    tbm[tid + i * kThreads] = 0u;
+    cbm[tid + i * kThreads] = 0u;
+  }
+  __syncthreads();
+  if (touched) {
+    places([&](int, int32_t id) { atomicOr(&tbm[id >> 5], 1u << (id & 31)); });
+    __syncthreads();
+  }
+  // Calls f(token, keys, bits) for each quad of untouched tokens, with every
+  // thread of a wave (key 0: past the row, masked or touched).
+  auto quads = [&](auto f) {
+    constexpr int U = 4;
+#pragma unroll 1
+    for (int64_t i0 = 4 * tid; i0 - 4 * tid < r.V; i0 += 4 * kThreads * U) {
+      uint32_t w[U][4], ok[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int64_t i = i0 + 4 * kThreads * u;
+        wide_quad<DT>(r, i, w[u]);
+        ok[u] = i < r.V ? (r.allow ? r.allow[i >> 5] >> (i & 31) : 0xFu) : 0u;
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int64_t i = i0 + 4 * kThreads * u;
+        if (touched && i < r.V) ok[u] &= ~(tbm[i >> 5] >> (i & 31));
+        uint32_t key[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) key[e] = f32_key(w[u][e], (ok[u] >> e) & 1u);
+        f(i, key, w[u]);
+      }
+    }
+  };
+  uint32_t kth = 0u, mask = 0u;
+  long long rem = k;
+#pragma unroll 1
+  for (int shift = 24; shift >= 0; shift -= 8) {
+    *reinterpret_cast<uint4*>(&t.hist[wave][4 * lane]) = make_uint4(0u, 0u, 0u, 0u);
+    wave_lds_sync();
+    // A wave's keys mostly share a bin in the upper passes: the first lane's
+    // bin is added once.
+    auto count = [&](uint32_t key) {
+      const bool on = key != 0u && (key & mask) == kth;
+      const unsigned long long m = __ballot(on);
+      if (m == 0ull) return;
+      const uint32_t bin = (key >> shift) & 0xFFu;
+      const int first = __ffsll((long long)m) - 1;
+      const uint32_t b0 = lane_value(bin, first);
+      const unsigned long long same = __ballot(on && bin == b0);
+      if (lane == first) atomicAdd(&t.hist[wave][b0], (uint32_t)__popcll(same));
+      else if (on && bin != b0) atomicAdd(&t.hist[wave][bin], 1u);
+    };
+    quads([&](int64_t, const uint32_t key[4], const uint32_t*) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) count(key[e]);
+    });
+    if (touched)
+      places([&](int at, int32_t) {
+        const double x = tv[at];
+        const uint32_t key = x > -(double)INFINITY ? wide_floor_key(x) : 0u;
+        if (key != 0u && (key & mask) == kth) atomicAdd(&t.hist[wave][(key >> shift) & 0xFFu], 1u);
+      });
+    __syncthreads();
+    long long above;
+    const int b = f32_pick(t, rem, above);  // uniform
+    __syncthreads();
+    if (b < 0) return -1;  // fewer than k finite tokens
+    kth |= (uint32_t)b << shift;
+    mask |= 0xFFu << shift;
+    rem -= above;
+  }
+  // Values so close below the k-th that (v - M) / T may tie with its own
+  // belong to its tie group, which the list cuts by index (sampling.py:89-91).
+  {
+    const double v = (double)wide_key_value(kth);
+    kth = wide_floor_key(v - fabs(M - v) * 0x1p-50);
+  }
+  quads([&](int64_t i, const uint32_t key[4], const uint32_t*) {
+    uint32_t sel = 0u;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) sel |= key[e] >= kth ? 1u << e : 0u;
+    if (sel) atomicOr(&cbm[i >> 5], sel << (i & 31));
+  });
+  if (touched)
+    places([&](int at, int32_t id) {
+      const double x = tv[at];
+      if (x > -(double)INFINITY && wide_floor_key(x) >= kth) atomicOr(&cbm[id >> 5], 1u << (id & 31));
+    });
+  __syncthreads();
+  long long nc;
+  {
+    const uint4 q = *(const uint4*)&cbm[4 * tid];
+    const uint32_t c0 = __popc(q.x), c1 = __popc(q.y), c2 = __popc(q.z), c3 = __popc(q.w);
+    const long long ex = block_exclusive_scan_i64((long long)(c0 + c1 + c2 + c3), bs, nc);
+    if (nc > kF32Cap) return -1;
+    uint32_t b = (uint32_t)ex;
+    base[4 * tid] = (uint16_t)b;
+    base[4 * tid + 1] = (uint16_t)(b += c0);
+    base[4 * tid + 2] = (uint16_t)(b += c1);
+    base[4 * tid + 3] = (uint16_t)(b += c2);
+  }
+  __syncthreads();
+  const double T = r.pol.temperature;
+  auto place = [&](int64_t i, double v) {
+    const uint32_t b = (uint32_t)(i & 31);
+    const int at = (int)base[i >> 5] + __popc(cbm[i >> 5] & ((1u << b) - 1u));
+    t.cz[at] = (v - M) / T;  // sampling.py:86-88, true division
+    t.cid[at] = (int32_t)i;
+  };
+  quads([&](int64_t i, const uint32_t key[4], const uint32_t* w) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (key[e] >= kth) place(i + e, (double)__uint_as_float(w[e]));
+  });
+  // A token's value is at one place; its other places hold -inf.
+  if (touched)
+    places([&](int at, int32_t id) {
+      const double x = tv[at];
+      if (x > -(double)INFINITY && wide_floor_key(x) >= kth) place(id, x);
+    });
+  __syncthreads();
+  return (int)nc;
+}
+
+// The candidates of a top-k row, or -1 with the reason.
+template <int DT>
+__device__ __forceinline__ int wide_candidates(const RowSpec& r, const WideLayout& L, char* ws, double M, long long k,
+                                               F32Shared& shu, int& why) {
+  int nc = wide_candidates_prefix<DT>(r, L, ws, M, k, shu);
+  if (nc < 0) nc = wide_candidates_exact<DT>(r, L, ws, M, k, shu);  // uniform
+  if (nc < 0) why = kHandCapacity;
+  return nc;
 }
 
 // ---------------------------------------------------------------------------
