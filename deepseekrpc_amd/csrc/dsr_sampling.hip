@@ -320,8 +320,8 @@ __global__ __launch_bounds__(kThreads) void k_wide_topk(Src src, int others, uns
   int64_t n = 0;
   int st = -1;
   if (kind == kWideTopK || kind == kWideGreedy) {
-    double f;
-    const WideRow w = wide_row_of<false>(L, ws, r, f);
+    double f, m;
+    const WideRow w = wide_row_of<false>(L, ws, r, f, m);
     if (w.bad) {
       why = kHandInvalid;
     } else if (kind == kWideGreedy) {
@@ -375,7 +375,7 @@ __global__ __launch_bounds__(kThreads) void k_wide_draw(Src src, int others, uns
       int32_t ic = INT32_MAX;
       long long npos = 0;
       const WideKeep every{w.M, r.pol.temperature, 1.0 / r.pol.temperature, -INFINITY, r.pol.min_p, INT32_MAX};
-      why = wide_whole<DT>(r, L, ws, w, sh, every, vc, ic, Sk, npos, flags);
+      why = wide_whole(r, L, ws, w, sh, every, vc, ic, Sk, npos, flags);
       if (why == 0) {
         int st = Sk > 0.0 ? DSR_OK : DSR_E_NO_MASS;
         int64_t token = -1;

@@ -14,13 +14,13 @@
 //                   adjusted values go to the row's workspace.  Top-k rows:
 //                   the 16-bit key prefix of every 16-token group's maximum.
 //                   Whole rows: sum exp((v - m) / T) in float64 and the mass
-//                   per 1,024 half-binade blocks of the order key, relative
-//                   to the slice's own maximum m (the row's is not known yet).
+//                   per 1,024 bins of m - v, relative to the slice's own
+//                   maximum m (the row's is not known yet).
 //   k_wide_bracket  one workgroup per whole row: the row's maximum and sum, and
-//                   from the slices' block masses the blocks that can hold
-//                   the min-p and top-p boundaries.
-//   k_wide_collect  filtered whole rows: each slice lists its tokens in those
-//                   blocks and sums the tokens above them.
+//                   from the slices' bin masses the values between which
+//                   the min-p and top-p boundaries lie.
+//   k_wide_collect  filtered whole rows: each slice lists its tokens between
+//                   those values and sums the tokens above them.
 //   k_wide_topk     one workgroup per top-k row: the k-th largest group
 //                   prefix bounds the k-th largest token from below (the
 //                   groups and touched tokens partition the row), only the
@@ -41,7 +41,7 @@
 // 64 bf16 rows, top-k 50, 4,096-token histories 953 us, now 28; 32 FP32 rows
 // of mixed whole policies with distributions 297, now 76.
 //
-// Block masses only bracket a boundary (they carry 36-bit fixed point and
+// Bin masses only bracket a boundary (they carry 36-bit fixed point and
 // FP32 rounding, and the bracket allows for both); every decision is made
 // again in float64 from the listed tokens' own exps and float64 sums, in a
 // fixed order.  Rows outside these limits (and invalid ones, whose status
@@ -62,9 +62,9 @@ constexpr int kWideSlice = kWideThreads * kWidePer;       // 8,192
 constexpr int kWideMaxSlices = 16;
 constexpr int kWideGroup = 16;                            // tokens per group maximum
 constexpr int kWideGroups = kWideSlice / kWideGroup;      // 512 per slice
-constexpr int kWideBlocks = 1024;                         // order-key blocks: key >> 22
+constexpr int kWideBins = 1024;                           // bins of (maximum - value)
 constexpr int kWideCand = 2048;                           // listed tokens per slice, at most (WideLayout::cand_cap)
-constexpr int kWideFine = kThreads;                       // tokens of the boundary bin, resolved exactly (one per thread)
+constexpr int kWideFine = kThreads;                       // tokens of the cut's sub-bin, resolved exactly (one per thread)
 constexpr int kWidePrefix = DSR_MAX_DRAFTS;               // touched places of a tentative prefix
 constexpr int kWideHistCopies = 2;
 static_assert((int64_t)kWideMaxSlices * kWideSlice >= DSR_MAX_VOCAB, "the slices cover the vocabulary");
@@ -100,8 +100,8 @@ struct WideRow {      // one row, from k_wide_bracket
   int32_t first;      // greedy rows: first index holding M
   int32_t npos;       // whole rows with no filter: finite tokens
   int32_t bad;        // invalid: the general path reports it
-  int32_t hi, plo, phi, mlo, mhi;  // WideBracket
   int32_t pad;
+  double hi, plo, phi, mlo, mhi;  // WideBracket
 };
 
 struct WideDec {      // one whole row's kept set, from k_wide_draw
@@ -124,7 +124,7 @@ struct WideLayout {
   __host__ __device__ size_t row_off() const { return dec_off() + 64; }
   __host__ __device__ size_t scale_off() const { return row_off() + 128; }
   __host__ __device__ size_t hist_off() const { return scale_off() + 128; }
-  __host__ __device__ size_t group_off() const { return hist_off() + (size_t)nS * kWideBlocks * sizeof(float); }
+  __host__ __device__ size_t group_off() const { return hist_off() + (size_t)nS * kWideBins * sizeof(float); }
   __host__ __device__ size_t cand_off() const { return group_off() + (size_t)nS * kWideGroups * sizeof(uint16_t); }
   __host__ __device__ size_t touch_off() const { return cand_off() + (size_t)nS * cand_cap() * 12; }
   // Touched tokens the rest of the row's workspace holds (a float64 value and a 16-bit key each).
@@ -344,20 +344,8 @@ __device__ __forceinline__ void wide_touched_each(const RowSpec& r, int e0, int 
   for (int b = b0 + (int)threadIdx.x; b < b1; b += STRIDE) f((int)r.pen_n + kWidePrefix + b, r.bias_ids[b]);
 }
 
-// The same by one wave.
-template <class F>
-__device__ __forceinline__ void wide_touched_wave(const RowSpec& r, const WideRec& rc, int64_t lo, int64_t hi, F f) {
-  const int l = lane_id();
-  for (int e = rc.e0 + l; e < rc.e1; e += 64) f(e, r.pen_ids[e]);
-  if (l < r.prefix_n) {
-    const int32_t id = r.prefix[l];
-    if (id >= lo && id < hi) f((int)r.pen_n + l, id);
-  }
-  for (int b = rc.b0 + l; b < rc.b1; b += 64) f((int)r.pen_n + kWidePrefix + b, r.bias_ids[b]);
-}
-
-// Order key of the largest float not above v (finite v), as f32_key orders floats.
-__device__ __forceinline__ uint32_t wide_floor_key(double v) {
+// The largest float not above v.
+__device__ __forceinline__ float wide_floor(double v) {
   float f = (float)v;
   if ((double)f > v) {  // step one float down
     uint32_t b = __float_as_uint(f);
@@ -366,21 +354,29 @@ __device__ __forceinline__ uint32_t wide_floor_key(double v) {
     else b += 1u;
     f = __uint_as_float(b);
   }
-  return f32_key(__float_as_uint(f), true);
+  return f;
 }
+
+// Its order key (finite v), as f32_key orders floats.
+__device__ __forceinline__ uint32_t wide_floor_key(double v) { return f32_key(__float_as_uint(wide_floor(v)), true); }
 
 // The float an order key (f32_key) stands for.
 __device__ __forceinline__ float wide_key_value(uint32_t k) {
   return __uint_as_float((k & 0x80000000u) ? (k & 0x7FFFFFFFu) : ~k);
 }
 
-// The block of a value: half a binade of the order key.  -0 falls one block
-// below +0 here (their tie group is listed whole: wide_bracket).
-__device__ __forceinline__ int wide_block(uint32_t key32) { return (int)(key32 >> 22); }
-__device__ __forceinline__ int wide_block_f(float v) {
-  const uint32_t b = __float_as_uint(v);
-  return (int)((b >> 22) ^ (((uint32_t)((int32_t)b >> 31) >> 22) | 0x200u));
+// Bins per logit: a whole row's masses are counted by (maximum - value), as its
+// law depends on that alone, in bins of T / 32, or sqrt(T) / 32 above T = 1
+// (of T / 32 a hot row would fill few).  So 1,024 bins reach 32 nats down, where
+// a token's mass is 1e-14, and 32 / sqrt(T) nats in hot rows, whose logits
+// span fewer; what lies lower shares the last bin.
+__device__ __forceinline__ double wide_per_logit(const dsr_policy_t& p) {
+  const double T = fmax(p.temperature, 1e-6);
+  return 32.0 / (T > 1.0 ? sqrt(T) : T);
 }
+
+// The bin of distance y (in bins, >= 0; a NaN: the last).
+__device__ __forceinline__ int wide_bin(double y) { return (int)fmin(y, (double)(kWideBins - 1)); }
 
 // a / T, rounded as the IEEE quotient (sampling.py:88 divides), from iT = 1 / T
 // rounded: a product and one correction by its exact remainder (P. W.
@@ -425,13 +421,13 @@ struct WideWaveRec {   // one wave's part of a slice
   uint32_t n, csum, bad, pad;
 };
 
-// A token's part of a block's 64-bit word: the bits of the double 2^52 + 2^50
+// A token's part of a bin's 64-bit word: the bits of the double 2^52 + 2^50
 // + mass * 2^36.  A slice's masses sum below 2^50, so the low 50 bits of a
 // word are their sum (the others mean nothing).
 constexpr double kWideOne = 0x1p52 + 0x1p50;
 struct WideHist {
   // The copies start on different banks.
-  unsigned long long w[kWideHistCopies][kWideBlocks + 8];
+  unsigned long long w[kWideHistCopies][kWideBins + 8];
 };
 
 template <bool WHOLE>
@@ -472,7 +468,7 @@ __global__ __launch_bounds__(kWideThreads) void k_wide_scan(Src src, int nS, int
 
   const bool whole = WHOLE && kind == kWideWhole;
   const bool nof = wide_nofilter(p);
-  const bool hist = whole && !nof;  // only filtered rows look for a block
+  const bool hist = whole && !nof;  // only filtered rows look for a bin
   if (t < kWideSlice / 32) {
     sh.tbits[t] = 0u;
     sh.kbits[t] = 0u;
@@ -764,22 +760,24 @@ __global__ __launch_bounds__(kWideThreads) void k_wide_scan(Src src, int nS, int
   }
   if constexpr (WHOLE) {
     if (whole && M > -(double)INFINITY) {
-      const double iT = 1.0 / p.temperature;
+      const double iT = 1.0 / p.temperature, per = wide_per_logit(p);
       double sum = 0.0;
       unsigned long long* h = sh.hist.w[t & (kWideHistCopies - 1)];
-      auto add = [&](double x, int block) {  // x = -inf adds 0, to block 1 (which holds no finite value)
+      auto add = [&](double x) {  // x = -inf adds 0
         const double e = wide_exp(wide_over(x - M, p.temperature, iT));
         sum += e;
-        if (hist) atomicAdd(&h[block], (unsigned long long)__double_as_longlong(__builtin_fma(e, 0x1p36, kWideOne)));
+        // A smaller mass is 0 in these units; many such tokens share the last bin.
+        if (hist && e > 0x1p-37)
+          atomicAdd(&h[wide_bin((M - x) * per)], (unsigned long long)__double_as_longlong(__builtin_fma(e, 0x1p36, kWideOne)));
       };
 #pragma unroll
       for (int k = 0; k < kWidePer; ++k) {
-        add((double)v[k], wide_block_f(v[k]));
+        add((double)v[k]);
         if (k % 4 == 3) __builtin_amdgcn_sched_barrier(0);  // four exps in flight: more cost registers
       }
       if (touched) {
         auto again = [&](double x) {
-          if (x > -(double)INFINITY) add(x, wide_block(wide_floor_key(x)));
+          if (x > -(double)INFINITY) add(x);
         };
         if (simple) {
 #pragma unroll
@@ -795,7 +793,7 @@ __global__ __launch_bounds__(kWideThreads) void k_wide_scan(Src src, int nS, int
 #pragma unroll
       for (int q = 0; q < kWideWaves; ++q) o.sum += sh.rs[q];
       if (hist) {
-        float4* ho = (float4*)(L.hist(ws) + s * kWideBlocks) + t;  // blocks 4t .. 4t + 3
+        float4* ho = (float4*)(L.hist(ws) + s * kWideBins) + t;  // bins 4t .. 4t + 3
         float f[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
@@ -813,9 +811,9 @@ __global__ __launch_bounds__(kWideThreads) void k_wide_scan(Src src, int nS, int
 
 // ---------------------------------------------------------------------------
 // What the slices' records say about a row, in every lane (uniform).  WHOLE:
-// S, and lane l's factor exp((m - M) / T) of slice l.
+// S, lane l's factor exp((m - M) / T) of slice l, and that slice's maximum.
 template <bool WHOLE>
-__device__ __forceinline__ WideRow wide_row_of(const WideLayout& L, char* ws, const RowSpec& r, double& factor) {
+__device__ __forceinline__ WideRow wide_row_of(const WideLayout& L, char* ws, const RowSpec& r, double& factor, double& m) {
   const int l = lane_id();
   WideRow o;
   WideRec x;
@@ -838,9 +836,10 @@ __device__ __forceinline__ WideRow wide_row_of(const WideLayout& L, char* ws, co
     off = off || x.e0 != (l ? pe1 : 0) || x.b0 != (l ? pb1 : 0);
     if (l == L.nS - 1) off = off || x.e1 != (int)r.pen_n || x.b1 != (int)r.bias_n;
   }
+  m = x.m;
   o.bad = __ballot(off) != 0ull || csum > DSR_MAX_COUNT || !(o.M > -(double)INFINITY);
   o.S = 0.0;
-  o.hi = o.plo = o.phi = o.mlo = o.mhi = o.pad = 0;
+  o.pad = 0;
   if constexpr (WHOLE) {
     o.vmin = lane_value(row_reduce(x.vmin, OpMin()), 0);
     o.npos = (int32_t)lane_value(row_reduce((uint32_t)x.npos, OpSum()), 0);
@@ -859,100 +858,125 @@ __device__ __forceinline__ bool wide_spread(const WideRow& w, const dsr_policy_t
 // ---------------------------------------------------------------------------
 // Step 2.
 
-// Blocks that can hold the boundaries of a filtered whole row.  Tokens in
-// blocks above `hi` are kept; those in [plo, phi] and [mlo, mhi] are listed;
-// those between mhi and plo count in the min-p mass only.
+// The values between which the boundaries of a filtered whole row lie.  Tokens
+// above `hi` are kept; those in [plo, phi] and [mlo, mhi] are listed; those
+// between mhi and plo count in the min-p mass only.  V: double, or float for
+// the same tests on untouched tokens.
+template <class V>
 struct WideBracket {
-  int hi;
-  int plo, phi;  // top-p (1024, -1: none)
-  int mlo, mhi;  // min-p (1024, -1: none)
-  __device__ __forceinline__ bool kept(int b) const { return b > hi; }
-  __device__ __forceinline__ bool listed(int b) const { return (b >= plo && b <= phi) || (b >= mlo && b <= mhi); }
-  __device__ __forceinline__ bool middle(int b) const { return b < plo && b > mhi; }
+  V hi;
+  V plo, phi;  // top-p (inf, -inf: none)
+  V mlo, mhi;  // min-p (inf, -inf: none)
+  __device__ __forceinline__ bool kept(V v) const { return v > hi; }
+  __device__ __forceinline__ bool listed(V v) const {
+    return (bool)(((int)(v >= plo) & (int)(v <= phi)) | ((int)(v >= mlo) & (int)(v <= mhi)));
+  }
+  __device__ __forceinline__ bool middle(V v) const { return (bool)((int)(v < plo) & (int)(v > mhi)); }
 };
 
-constexpr int kBracketThreads = kWideBlocks / 2;
+__device__ __forceinline__ WideBracket<float> wide_bracket_f(const WideBracket<double>& b) {
+  return {wide_floor(b.hi), -wide_floor(-b.plo), wide_floor(b.phi), -wide_floor(-b.mlo), wide_floor(b.mhi)};
+}
+
+constexpr int kBracketThreads = kWideBins / 2;
 
 struct WideBracketShared {
   double blk[kBracketThreads / 64];
-  double pre[kWideBlocks];  // mass per block, inclusive from the top
+  double pre[kWideBins];  // running mass, see wide_bracket
   double scale[kWideMaxSlices];
+  int off[kWideMaxSlices];
   int b[2];
 };
 
-// Relative and absolute slack of a running block mass: FP32 block sums and
+// Relative and absolute slack of a running bin mass: FP32 bin sums and
 // 2^-36 fixed-point masses (an absolute 2^-37 per token of a row whose
 // largest mass is 1).
 constexpr double kWideRel = 0x1p-20;
 constexpr double kWideAbs = 0x1p-18;
 
 // Every thread of the workgroup calls.
-__device__ __forceinline__ WideBracket wide_bracket(const WideLayout& L, char* ws, const RowSpec& r, const WideRow& w,
-                                                    WideBracketShared& sh) {
+//
+// With y = (M - v) * per, a token of slice s in its bin j has y in [d + j, d + j
+// + 1), d = (M - m_s) * per.  R(b) = the mass of the bins with floor(d) + j <= b
+// is at least the mass of the tokens with y < b + 1, and at most that of those
+// with y < b + 2.  Bins widened by a hundredth take care of the rounding of y.
+__device__ __forceinline__ WideBracket<double> wide_bracket(const WideLayout& L, char* ws, const RowSpec& r, const WideRow& w,
+                                                            WideBracketShared& sh) {
   const int t = threadIdx.x;
   const dsr_policy_t& p = r.pol;
   const float* h = L.hist(ws);
-  // Thread t holds blocks 1023 - 2t and 1022 - 2t.
-  const int b0 = kWideBlocks - 1 - 2 * t;
+  const double per = wide_per_logit(p);
+  constexpr int kLast = kWideBins - 2;  // the last bin has no end
+  const int b0 = 2 * t;                 // this thread's bins: b0, b0 + 1
   double x0 = 0.0, x1 = 0.0;
   {
     // Slices past the row's read its last one again (a branch would make each
     // load wait for the one before).  Theirs count nothing, nor do those of a
     // slice without a finite token, which k_wide_scan leaves unwritten: a
     // factor of 0 is selected on, for what lies there may be a NaN.
-    float2 q[kWideMaxSlices];
+    float q[kWideMaxSlices][2];
 #pragma unroll
-    for (int s = 0; s < kWideMaxSlices; ++s) q[s] = *(const float2*)(h + min(s, L.nS - 1) * kWideBlocks + b0 - 1);
+    for (int s = 0; s < kWideMaxSlices; ++s) {
+      const float* hs = h + min(s, L.nS - 1) * kWideBins;
+      const int j = b0 - sh.off[s];
+      q[s][0] = hs[max(j, 0)];
+      q[s][1] = hs[max(j + 1, 0)];
+    }
 #pragma unroll
     for (int s = 0; s < kWideMaxSlices; ++s) {
       const double f = sh.scale[s];
-      x0 += f != 0.0 ? f * (double)q[s].y : 0.0;
-      x1 += f != 0.0 ? f * (double)q[s].x : 0.0;
+      const int j = b0 - sh.off[s];
+      x0 += f != 0.0 && j >= 0 ? f * (double)q[s][0] : 0.0;
+      x1 += f != 0.0 && j + 1 >= 0 ? f * (double)q[s][1] : 0.0;
     }
   }
   const double incl = wave_scan_dpp(x0 + x1);
   if (lane_id() == 63) sh.blk[wave_id()] = incl;
-  if (t < 2) sh.b[t] = -1;
+  if (t < 2) sh.b[t] = INT_MAX;
   lds_barrier();
   double base = 0.0;
   for (int q = 0; q < wave_id(); ++q) base += sh.blk[q];
-  const double i1 = base + incl, i0 = i1 - x1;  // inclusive from the top through b0 - 1 and b0
+  const double i1 = base + incl, i0 = i1 - x1;  // R(b0 + 1), R(b0)
   sh.pre[b0] = i0;
-  sh.pre[b0 - 1] = i1;
+  sh.pre[b0 + 1] = i1;
   lds_barrier();
-  WideBracket o;
-  o.plo = o.mlo = kWideBlocks;
-  o.phi = o.mhi = -1;
+  WideBracket<double> o;
+  o.plo = o.mlo = INFINITY;
+  o.phi = o.mhi = -INFINITY;
   double slo = w.S, shi = w.S;
   if (p.min_p != 0.0) {  // kept: exp((v - M) / T) >= min_p
     const double ln = log(p.min_p);
     const double span = p.temperature * ln, e = 1e-9 * (fabs(span) + fabs(w.M)) + 1e-300;
-    o.mlo = wide_block(wide_floor_key(w.M + span - e));
-    o.mhi = wide_block(wide_floor_key(w.M + span + e));
-    shi = fmin(shi, sh.pre[o.mlo] * (1.0 + kWideRel) + kWideAbs);
-    slo = o.mhi + 1 < kWideBlocks ? fmax(sh.pre[o.mhi + 1] * (1.0 - kWideRel) - kWideAbs, 0.0) : 0.0;
+    o.mlo = w.M + span - e;
+    o.mhi = w.M + span + e;
+    const double far = (w.M - o.mlo) * per + 0.01, sure = fmax((w.M - o.mhi) * per - 0.01, 0.0);
+    if (far < (double)kLast) shi = fmin(shi, sh.pre[(int)far] * (1.0 + kWideRel) + kWideAbs);
+    const int b = (int)fmin(sure, (double)kLast) - 2;
+    slo = fmax(b >= 0 ? sh.pre[b] * (1.0 - kWideRel) - kWideAbs : 0.0, 1.0);  // the maximum's mass is 1
   }
   o.hi = o.mhi;
   if (p.top_p < 1.0) {
     const double plo = p.top_p * slo * (1.0 - kWideRel) - kWideAbs, phi = p.top_p * shi * (1.0 + kWideRel) + kWideAbs;
-    // The highest block whose running mass can reach the boundary, and the
-    // first whose running mass must have passed it (none: the lowest).
-    auto up = [&](double in) { return in > 0.0 && in * (1.0 + kWideRel) + kWideAbs >= plo; };
+    // The first bin that can hold the cut, and the first whose R must have passed it.
+    auto up = [&](double in) { return in * (1.0 + kWideRel) + kWideAbs >= plo; };
     auto dn = [&](double in) { return in * (1.0 - kWideRel) - kWideAbs >= phi; };
 #pragma unroll
     for (int q = 0; q < 2; ++q) {
-      const int b = b0 - q;
-      const double in = q ? i1 : i0, ex = b + 1 < kWideBlocks ? sh.pre[b + 1] : 0.0;
-      if (up(in) && !up(ex)) atomicMax(&sh.b[0], b);
-      if (dn(in) && !dn(ex)) atomicMax(&sh.b[1], b);
+      const int b = b0 + q;
+      if (b > kLast) continue;
+      const double in = q ? i1 : i0;
+      if (up(in) && (b == 0 || !up(sh.pre[b - 1]))) atomicMin(&sh.b[0], b);
+      if (dn(in) && (b == 0 || !dn(sh.pre[b - 1]))) atomicMin(&sh.b[1], b);
     }
     lds_barrier();
-    o.phi = sh.b[0] < 0 ? kWideBlocks - 1 : sh.b[0];
-    o.plo = sh.b[1] < 0 ? 0 : sh.b[1];
-    if (o.plo > o.phi) o.plo = o.phi;
-    if (o.phi == 511) o.phi = 512;  // -0 ties with +0 one block above
-    if (o.plo == 512) o.plo = 511;
-    o.hi = o.phi > o.mhi ? o.phi : o.mhi;
+    const int bl = min(sh.b[0], kLast + 1), bh = sh.b[1];
+    o.phi = bl == 0 ? INFINITY : w.M - ((double)bl - 0.01) / per;
+    o.plo = bh == INT_MAX ? -INFINITY : w.M - ((double)bh + 2.01) / per;
+    if (!(fabs(w.M) * 0x1p-48 <= 0.005 / per)) {  // a bin is no wider than the rounding of a value
+      o.phi = INFINITY;
+      o.plo = -INFINITY;
+    }
+    o.hi = fmax(o.phi, o.mhi);
   }
   return o;
 }
@@ -969,24 +993,26 @@ __global__ __launch_bounds__(kBracketThreads) void k_wide_bracket(Src src) {
   if (kind != kWideWhole && kind != kWideGreedy) return;
   char* ws = src.ws(d);
   WideRow w;
-  double f = 0.0;
-  if (kind == kWideGreedy) w = wide_row_of<false>(L, ws, r, f);
-  else w = wide_row_of<true>(L, ws, r, f);
+  double f = 0.0, m;
+  if (kind == kWideGreedy) w = wide_row_of<false>(L, ws, r, f, m);
+  else w = wide_row_of<true>(L, ws, r, f, m);
   if (threadIdx.x < kWideMaxSlices) {
+    const double d = (w.M - m) * wide_per_logit(r.pol);
     sh.scale[threadIdx.x] = f;
+    sh.off[threadIdx.x] = d < (double)kWideBins ? (int)d : kWideBins;  // no finite token: factor 0
     L.scale(ws)[threadIdx.x] = f;
   }
   if (kind == kWideWhole && !w.bad && !wide_nofilter(r.pol)) {  // uniform
     lds_barrier();
-    const WideBracket B = wide_bracket(L, ws, r, w, sh);
+    const WideBracket<double> B = wide_bracket(L, ws, r, w, sh);
     w.hi = B.hi;
     w.plo = B.plo;
     w.phi = B.phi;
     w.mlo = B.mlo;
     w.mhi = B.mhi;
   } else {  // every token kept (read for rows with no filter)
-    w.hi = w.phi = w.mhi = -1;
-    w.plo = w.mlo = kWideBlocks;
+    w.hi = w.phi = w.mhi = -INFINITY;
+    w.plo = w.mlo = INFINITY;
   }
   if (threadIdx.x == 0) {
     WideRow* o = L.row(ws);
@@ -1027,7 +1053,8 @@ __global__ __launch_bounds__(kWideThreads) void k_wide_collect(Src src, int nS) 
   const WideRow w = *L.row(ws);
   if (w.bad) return;  // uniform
   if (wide_nofilter(p) && !wide_spread(w, p)) return;  // the records decide it
-  const WideBracket B{w.hi, w.plo, w.phi, w.mlo, w.mhi};
+  const WideBracket<double> B{w.hi, w.plo, w.phi, w.mlo, w.mhi};
+  const WideBracket<float> F = wide_bracket_f(B);
   const double M = w.M;
   const int lo = s * kWideSlice, hi = lo + kWideSlice < (int)r.V ? lo + kWideSlice : (int)r.V;
   const bool touched = wide_touched(r);
@@ -1053,10 +1080,9 @@ __global__ __launch_bounds__(kWideThreads) void k_wide_collect(Src src, int nS) 
   uint32_t nm = 0u, sel = 0u;  // nm: uniform
 #pragma unroll
   for (int k = 0; k < kWidePer; ++k) {
-    const int b = wide_block_f(v[k]);
-    const bool f = ((ok >> k) & 1u) && v[k] > -INFINITY;
-    const bool sum = f && (B.kept(b) || (mids && B.middle(b)));
-    if (f && !B.kept(b) && B.listed(b)) sel |= 1u << k;
+    const bool f = ((ok >> k) & 1u) && v[k] > -INFINITY, kp = F.kept(v[k]);
+    const bool sum = f && (kp || (mids && F.middle(v[k])));
+    if (f && !kp && F.listed(v[k])) sel |= 1u << k;
     const unsigned long long bal = __ballot(sum);
     if (sum) mv[nm + lanes_below(bal)] = v[k];
     nm += (uint32_t)__popcll(bal);
@@ -1071,15 +1097,14 @@ __global__ __launch_bounds__(kWideThreads) void k_wide_collect(Src src, int nS) 
     npos += k && e > 0.0 ? 1u : 0u;
     mid += k ? 0.0 : e;
   };
-  for (uint32_t i = (uint32_t)lane; i < nm; i += 64u) add((double)mv[i], B.kept(wide_block_f(mv[i])));
+  for (uint32_t i = (uint32_t)lane; i < nm; i += 64u) add((double)mv[i], F.kept(mv[i]));
   if (touched)
     wide_touched_each<kWideThreads>(r, rc.e0, rc.e1, rc.b0, rc.b1, lo, hi, [&](int at, int32_t) {
       const double x = tv[at];
       if (!(x > -(double)INFINITY)) return;
-      const int b = wide_block(wide_floor_key(x));
-      const bool k = B.kept(b);
-      if (k || (mids && B.middle(b))) add(x, k);
-      if (!k && B.listed(b)) ++nt;
+      const bool k = B.kept(x);
+      if (k || (mids && B.middle(x))) add(x, k);
+      if (!k && B.listed(x)) ++nt;
     });
   // Listed tokens go to the slice's list in thread order (a fixed order).
   const uint32_t c = (uint32_t)__popc(sel) + nt;
@@ -1113,12 +1138,9 @@ __global__ __launch_bounds__(kWideThreads) void k_wide_collect(Src src, int nS) 
     if (nt)
       wide_touched_each<kWideThreads>(r, rc.e0, rc.e1, rc.b0, rc.b1, lo, hi, [&](int at, int32_t id) {
         const double x = tv[at];
-        if (x > -(double)INFINITY) {
-          const int b = wide_block(wide_floor_key(x));
-          if (!B.kept(b) && B.listed(b)) {
-            ov[at0] = x;
-            oi[at0++] = id;
-          }
+        if (x > -(double)INFINITY && !B.kept(x) && B.listed(x)) {
+          ov[at0] = x;
+          oi[at0++] = id;
         }
       });
   }
@@ -1155,9 +1177,7 @@ struct WideItem {  // a token of the boundary bin
 };
 
 struct WideCut {
-  unsigned long long bm[kWideBlocks];  // fixed-point mass per sub-bin of the listed blocks
-  uint32_t bn[kWideBlocks];            // and the tokens in it
-  uint32_t tb[kWideMaxSlices][kWideSlice / 32];  // touched tokens, per slice (a row read again)
+  unsigned long long bm[kWideBins];  // fixed-point mass per sub-bin of the listed values
   WideItem list[kWideFine];
   double sv[kWideFine], sm[kWideFine];  // the list in rank order, and its masses
   int32_t si[kWideFine];
@@ -1178,89 +1198,42 @@ struct WideDrawShared {
   double Ks[kWideMaxSlices];           // kept mass per slice
   double part[2][kWideMaxSlices];
   uint32_t cnt[2][kWideMaxSlices];
-  long long run;
   int nlist, bin, tok, margin;
   uint32_t close;
 };
 
-// Where a row's listed tokens are: in the lists of its slices, n in this
-// wave's, or, OVER, in the row itself.
-struct WideItems {
-  int n;
-  WideBracket B;
-};
-
-// Calls f(value, id, key) for the listed tokens of slice `wave` (each by one
-// lane, in a fixed order; eight list entries or four quads of the row in flight).
-template <int DT, bool OVER, class F>
-__device__ __forceinline__ void wide_listed(const RowSpec& r, const WideLayout& L, char* ws, int wave, const WideItems& it,
-                                            const WideCut& c, F f) {
-  if constexpr (!OVER) {
-    const int n = it.n, w = wave < L.nS ? wave : 0;  // n is 0 past the row's slices
-    const double* cv = L.cand_v(ws, w);
-    const int32_t* ci = L.cand_i(ws, w);
-    constexpr int U = 8;
-    for (int i0 = lane_id(); i0 < n; i0 += 64 * U) {
-      double v[U];
-      int32_t id[U];
+// Calls f(value, id) for the listed tokens of slice `wave` (lane-strided, a
+// fixed order; eight loads in flight).
+template <class F>
+__device__ __forceinline__ void wide_listed(const WideLayout& L, char* ws, int wave, int n, F f) {
+  const int w = wave < L.nS ? wave : 0;  // n is 0 past the row's slices
+  const double* cv = L.cand_v(ws, w);
+  const int32_t* ci = L.cand_i(ws, w);
+  constexpr int U = 8;
+  for (int i0 = lane_id(); i0 < n; i0 += 64 * U) {
+    double v[U];
+    int32_t id[U];
 #pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int i = min(i0 + 64 * u, n - 1);  // unbranched loads
-        v[u] = cv[i];
-        id[u] = ci[i];
-      }
-#pragma unroll
-      for (int u = 0; u < U; ++u)
-        if (i0 + 64 * u < n) f(v[u], id[u], wide_floor_key(v[u]));  // an untouched value is a float: its own key
+    for (int u = 0; u < U; ++u) {
+      const int i = min(i0 + 64 * u, n - 1);  // unbranched loads
+      v[u] = cv[i];
+      id[u] = ci[i];
     }
-  } else if (wave < L.nS) {
-    const int64_t lo = (int64_t)wave * kWideSlice, hi = lo + kWideSlice < r.V ? lo + kWideSlice : r.V;
-    const bool touched = wide_touched(r);
-    constexpr int U = 4;
-#pragma unroll 1
-    for (int64_t i0 = lo + 4 * lane_id(); i0 < hi; i0 += 256 * U) {
-      uint32_t w[U][4], ok[U];
 #pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int64_t i = i0 + 256 * u;
-        wide_quad<DT>(r, i, w[u]);  // slices start at multiples of 1,024: past this one lies the row's end
-        ok[u] = i < hi ? (r.allow ? r.allow[i >> 5] >> (i & 31) : 0xFu) : 0u;
-      }
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int64_t i = i0 + 256 * u;
-        if (touched && i < hi) ok[u] &= ~(c.tb[wave][(i - lo) >> 5] >> (i & 31));
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const float v = __uint_as_float(w[u][e]);
-          const int b = wide_block_f(v);
-          if (((ok[u] >> e) & 1u) && v > -INFINITY && !it.B.kept(b) && it.B.listed(b))
-            f((double)v, (int32_t)(i + e), f32_key(w[u][e], true));
-        }
-      }
-    }
-    if (touched) {
-      const double* tv = L.tv(ws);
-      wide_touched_wave(r, L.rec(ws)[wave], lo, hi, [&](int at, int32_t id) {
-        const double x = tv[at];
-        const uint32_t key = wide_floor_key(x);
-        const int b = wide_block(key);
-        if (x > -(double)INFINITY && !it.B.kept(b) && it.B.listed(b)) f(x, id, key);
-      });
-    }
+    for (int u = 0; u < U; ++u)
+      if (i0 + 64 * u < n) f(v[u], id[u]);
   }
 }
 
 // The min-p mass of a row (sampling.py:94-96: kept when r >= min_p * max(r)):
-// the mass above the listed blocks and between them, and the listed tokens
+// the mass above the listed values and between them, and the listed tokens
 // themselves.
-template <int DT, bool OVER>
-__device__ __forceinline__ double wide_minp_mass(const RowSpec& r, const WideLayout& L, char* ws, const WideItems& it,
-                                                 const WideSum& mine, WideDrawShared& sh, const WideKeep& K, unsigned& flags) {
+__device__ __forceinline__ double wide_minp_mass(const WideLayout& L, char* ws, int n, const WideSum& mine, WideDrawShared& sh,
+                                                 const WideKeep& K, unsigned& flags) {
   const int wave = __builtin_amdgcn_readfirstlane(wave_id());
   double s = 0.0;
   uint32_t close = 0u;
-  wide_listed<DT, OVER>(r, L, ws, wave, it, sh.c, [&](double v, int32_t, uint32_t) {
+  wide_listed(L, ws, wave, n, [&](double v, int32_t) {
     const double e = wide_exp(wide_over(v - K.M, K.T, K.iT));
     if (e > 0.0 && fabs(e - K.min_p) <= K.min_p * 0x1p-48) close = 1u;
     s += e < K.min_p ? 0.0 : e;
@@ -1277,70 +1250,55 @@ __device__ __forceinline__ double wide_minp_mass(const RowSpec& r, const WideLay
 
 // The top-p cut of a whole row (sampling.py:97-102): the last kept token, by
 // value and index, into K, and the kept listed mass and positive count of
-// each slice into `s`, `c` of its wave.  `base` is the mass certainly kept
-// (nbase positive tokens), S the row's.  Returns 0 or the reason the general
-// path must decide the row.
-template <int DT, bool OVER>
-__device__ __forceinline__ int wide_cut(const RowSpec& r, const WideLayout& L, char* ws, const WideRow& row, const WideItems& it,
-                                        double base, long long nbase, double S, WideDrawShared& sh, const WideKeep& K, double& vc,
-                                        int32_t& ic, double& s, uint32_t& c, unsigned& flags) {
+// each slice into `s`, `c` of its wave.  `n` tokens are listed for this
+// wave's slice; `base` is the mass certainly kept (nbase positive tokens), S
+// the row's.  Returns 0 or the reason the general path must decide the row.
+__device__ __forceinline__ int wide_cut(const RowSpec& r, const WideLayout& L, char* ws, const WideRow& row, int n, double base,
+                                        long long nbase, double S, WideDrawShared& sh, const WideKeep& K, double& vc, int32_t& ic, double& s,
+                                        uint32_t& c, unsigned& flags) {
   const int t = threadIdx.x, lane = lane_id();
   const int wave = __builtin_amdgcn_readfirstlane(wave_id());
   const int nS = L.nS;
   BlockScratch& bs = sh.b;
-  // Fixed-point mass per sub-bin of the order keys of the listed blocks, then
-  // the bin that holds top_p * S.  OVER: a bin of more tokens than the list
-  // below takes is cut into 1,024 in turn, down to single keys.
-  const int blo = row.plo < row.mlo ? row.plo : row.mlo;
-  uint32_t klo = (uint32_t)blo << 22;
-  int shift = 12 + max(0, 32 - (int)__clz(max(0, row.hi - blo)));  // (hi - lo + 1) << 22 >> shift <= 1,024
+  // Fixed-point mass per sub-bin of the listed values, from the highest down
+  // (bins of the scan's width where they have no lower end), then the sub-bin
+  // that holds top_p * S.
+  const double top = fmin(row.hi, row.M), low = fmin(row.plo, row.mlo);
+  const double per = low > -(double)INFINITY ? 1023.0 / (top - low) : wide_per_logit(r.pol);
+  auto sub = [&](double v) { return wide_bin((top - v) * per); };
+  sh.c.bm[t] = 0ull;
+  if (t == 0) {
+    sh.bin = -1;
+    sh.nlist = 0;
+  }
+  lds_barrier();
+  wide_listed(L, ws, wave, n, [&](double v, int32_t) {
+    const double e = K.mass(v);
+    if (e > 0.0) atomicAdd(&sh.c.bm[sub(v)], (unsigned long long)(e * 0x1p45));
+  });
+  lds_barrier();
   const double P = r.pol.top_p * S;
-  long long run0 = (long long)(base * 0x1p45);  // mass above the bins
+  const long long b45 = (long long)(base * 0x1p45);
   long long tgt = (long long)(P * 0x1p45);
   if (tgt < 1) tgt = 1;
-  if (t == 0) sh.nlist = 0;
-  int bin;
-  for (;;) {  // uniform; at most four rounds
-    sh.c.bm[t] = 0ull;
-    if (OVER) sh.c.bn[t] = 0u;
-    if (t == 0) sh.bin = -1;
-    lds_barrier();
-    wide_listed<DT, OVER>(r, L, ws, wave, it, sh.c, [&](double v, int32_t, uint32_t key) {
-      const uint32_t b = (key - klo) >> shift;
-      if (OVER && (key < klo || b >= (uint32_t)kWideBlocks)) return;
-      const double e = K.mass(v);
-      if (OVER) atomicAdd(&sh.c.bn[b], 1u);
-      if (e > 0.0) atomicAdd(&sh.c.bm[b], (unsigned long long)(e * 0x1p45));
-    });
-    lds_barrier();
-    const long long mass = (long long)sh.c.bm[kWideBlocks - 1 - t];
-    long long tot;
-    const long long run = run0 + block_exclusive_scan_i64(mass, bs, tot);
-    if (run < tgt && tgt <= run + mass) {
-      sh.bin = kWideBlocks - 1 - t;
-      sh.run = run;
-    }
-    lds_barrier();
-    bin = sh.bin;
-    if (!OVER || bin < 0 || shift == 0 || sh.c.bn[bin] <= (uint32_t)kWideFine) break;
-    run0 = sh.run;
-    klo += (uint32_t)bin << shift;
-    shift = max(0, shift - 10);
-    lds_barrier();  // every thread has read the bin
-  }
+  const long long mass = (long long)sh.c.bm[t];
+  long long tot;
+  const long long run = b45 + block_exclusive_scan_i64(mass, bs, tot);
+  if (run < tgt && tgt <= run + mass) sh.bin = t;
+  lds_barrier();
   // A row that cannot be decided still takes every step below, with an empty list.
+  const int bin = sh.bin;
   int why = bin < 0 ? kHandCapacity : 0;  // rounding put the boundary outside the listed tokens
-  // The bin's tokens, and the mass and number of listed tokens above it.
-  const uint32_t kbin = klo + ((uint32_t)max(bin, 0) << shift);
+  // The sub-bin's tokens, and the mass and number of listed tokens above it.
   s = 0.0;
   c = 0u;
-  wide_listed<DT, OVER>(r, L, ws, wave, it, sh.c, [&](double v, int32_t id, uint32_t key) {
-    if (key < kbin) return;
-    if ((key - kbin) >> shift) {
+  wide_listed(L, ws, wave, n, [&](double v, int32_t id) {
+    const int b = sub(v);
+    if (b < bin) {
       const double e = K.mass(v);
       s += e;
       c += e > 0.0 ? 1u : 0u;
-    } else {
+    } else if (b == bin) {
       const int at = atomicAdd(&sh.nlist, 1);
       if (at < kWideFine) sh.c.list[at] = WideItem{v, id, 0};
     }
@@ -1402,7 +1360,7 @@ __device__ __forceinline__ int wide_cut(const RowSpec& r, const WideLayout& L, c
       if (v < vr) lower = fmax(lower, v);
       if (v > vk) upper = fmin(upper, v);
     };
-    wide_listed<DT, OVER>(r, L, ws, wave, it, sh.c, [&](double v, int32_t, uint32_t) { side(v); });
+    wide_listed(L, ws, wave, n, [&](double v, int32_t) { side(v); });
     const double* tv = L.tv(ws);
     for (int i = t; i < (int)r.pen_n; i += kThreads) side(tv[i]);
     if (t < r.prefix_n) side(tv[r.pen_n + t]);
@@ -1430,12 +1388,11 @@ __device__ __forceinline__ int wide_cut(const RowSpec& r, const WideLayout& L, c
 
 // A whole row: the kept set (K), the kept mass per slice (sh.Ks) and in all
 // (Sk), and its positive tokens.  Returns 0 or the reason the general path
-// must decide the row, kHandCapacity also when the slices' lists cannot.
-// Every thread of the 1,024 calls; wave w works on slice w.
-template <int DT, bool OVER>
-__device__ __forceinline__ int wide_whole_from(const RowSpec& r, const WideLayout& L, char* ws, const WideRow& row,
-                                               WideDrawShared& sh, const WideKeep& K, double& vc, int32_t& ic, double& Sk,
-                                               long long& npos, unsigned& flags) {
+// must decide the row.  Every thread of the 1,024 calls; wave w works on
+// slice w.
+__device__ __forceinline__ int wide_whole(const RowSpec& r, const WideLayout& L, char* ws, const WideRow& row,
+                                          WideDrawShared& sh, const WideKeep& K, double& vc, int32_t& ic, double& Sk, long long& npos,
+                                          unsigned& flags) {
   const int lane = lane_id();
   const int wave = __builtin_amdgcn_readfirstlane(wave_id());
   const dsr_policy_t& p = r.pol;
@@ -1448,27 +1405,18 @@ __device__ __forceinline__ int wide_whole_from(const RowSpec& r, const WideLayou
     mine.mid = lane_value(all.mid, wave);
     mine.ncand = (int32_t)lane_value((uint32_t)all.ncand, wave);
   }
-  const WideItems it{__builtin_amdgcn_readfirstlane(mine.ncand), WideBracket{row.hi, row.plo, row.phi, row.mlo, row.mhi}};
-  if (!OVER && __ballot(all.ncand > L.cand_cap())) return kHandCapacity;  // uniform over the workgroup
+  const int n = __builtin_amdgcn_readfirstlane(mine.ncand);
+  int why = __ballot(all.ncand > L.cand_cap()) ? kHandCapacity : 0;  // uniform over the workgroup
   const double base = lane_value(row_reduce(all.kept, OpSum()), 0);  // mass certainly kept, and its positive tokens
   const long long nbase = (long long)lane_value(row_reduce((uint32_t)all.npos, OpSum()), 0);
-  if (OVER && wide_touched(r) && wave < nS) {  // the wave's own slice
-    uint32_t* tb = sh.c.tb[wave];
-    const int64_t lo = (int64_t)wave * kWideSlice, hi = lo + kWideSlice < r.V ? lo + kWideSlice : r.V;
-    for (int i = lane; i < kWideSlice / 32; i += 64) tb[i] = 0u;
-    wave_lds_sync();
-    wide_touched_wave(r, L.rec(ws)[wave], lo, hi, [&](int, int32_t id) { atomicOr(&tb[(id - lo) >> 5], 1u << ((id - lo) & 31)); });
-    wave_lds_sync();
-  }
-  int why = 0;
   double s = 0.0;
   uint32_t c = 0u;
-  if (!nof) {
-    const double S = p.min_p != 0.0 ? wide_minp_mass<DT, OVER>(r, L, ws, it, mine, sh, K, flags) : row.S;
+  if (!nof && why == 0) {
+    const double S = p.min_p != 0.0 ? wide_minp_mass(L, ws, n, mine, sh, K, flags) : row.S;
     if (p.top_p < 1.0) {
-      why = wide_cut<DT, OVER>(r, L, ws, row, it, base, nbase, S, sh, K, vc, ic, s, c, flags);
+      why = wide_cut(r, L, ws, row, n, base, nbase, S, sh, K, vc, ic, s, c, flags);
     } else {  // min-p alone
-      wide_listed<DT, OVER>(r, L, ws, wave, it, sh.c, [&](double v, int32_t, uint32_t) {
+      wide_listed(L, ws, wave, n, [&](double v, int32_t) {
         const double e = K.mass(v);
         s += e;
         c += e > 0.0 ? 1u : 0u;
@@ -1489,28 +1437,6 @@ __device__ __forceinline__ int wide_whole_from(const RowSpec& r, const WideLayou
   for (int q = 0; q < nS; ++q) {
     Sk += sh.Ks[q];
     npos += sh.cnt[1][q];
-  }
-  return why;
-}
-
-// The same from the slices' lists, and again from the row where they cannot
-// tell: a slice lists more tokens than its list holds, or the cut's sub-bin more
-// than are ranked.  Blocks and sub-bins follow the logit itself, so that takes
-// logits with a common offset (N(0, 1) at +-70 and beyond) or nearly equal
-// ones.  A pass over a row of 129,280 is read at one workgroup's pace; the
-// general path, which such rows would take, needs 22.
-template <int DT>
-__device__ __forceinline__ int wide_whole(const RowSpec& r, const WideLayout& L, char* ws, const WideRow& row,
-                                          WideDrawShared& sh, const WideKeep& K, double& vc, int32_t& ic, double& Sk, long long& npos,
-                                          unsigned& flags) {
-  const unsigned flags0 = flags;
-  int why = wide_whole_from<DT, false>(r, L, ws, row, sh, K, vc, ic, Sk, npos, flags);
-  if (why == kHandCapacity && !wide_nofilter(r.pol)) {  // uniform
-    __syncthreads();  // every thread is done with the first attempt's LDS
-    if (threadIdx.x == 0) sh.close = 0u;
-    lds_barrier();
-    flags = flags0;
-    why = wide_whole_from<DT, true>(r, L, ws, row, sh, K, vc, ic, Sk, npos, flags);
   }
   return why;
 }

@@ -89,8 +89,8 @@ __global__ __launch_bounds__(kThreads) void k_wide_dist(WideVerifyRows src, int 
   int64_t onehot = -1;
   unsigned flags = 0;
   if (kind == kWideTopK || kind == kWideGreedy) {
-    double f;
-    const WideRow w = wide_row_of<false>(L, ws, r, f);
+    double f, m;
+    const WideRow w = wide_row_of<false>(L, ws, r, f, m);
     if (!w.bad && kind == kWideGreedy) {
       form = kFormOne;
       st = DSR_OK;
@@ -129,7 +129,7 @@ __global__ __launch_bounds__(kThreads) void k_wide_dist(WideVerifyRows src, int 
       int32_t ic = INT32_MAX;
       long long npos = 0;
       const WideKeep every{w.M, r.pol.temperature, 1.0 / r.pol.temperature, -INFINITY, r.pol.min_p, INT32_MAX};
-      why = wide_whole<DT>(r, L, ws, w, sh.w, every, vc, ic, Sk, npos, flags);
+      why = wide_whole(r, L, ws, w, sh.w, every, vc, ic, Sk, npos, flags);
       if (why == 0) {
         form = kFormWhole;
         st = Sk > 0.0 ? DSR_OK : DSR_E_NO_MASS;
