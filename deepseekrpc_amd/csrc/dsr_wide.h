@@ -112,7 +112,9 @@ struct WideDec {      // one whole row's kept set, from k_wide_draw
 
 static_assert(sizeof(WideRow) <= 128 && sizeof(WideDec) <= 64, "workspace layout");
 
-// Per-row workspace: every part a multiple of 16 bytes.
+// Per-row workspace: every part a multiple of 16 bytes.  After the records
+// come a top-k row's group keys, or another row's bin masses and lists, and in
+// the rest its touched tokens (TOP: a top-k row's).
 struct WideLayout {
   int64_t V;
   int nS;
@@ -123,29 +125,35 @@ struct WideLayout {
   __host__ __device__ size_t dec_off() const { return sum_off() + (((size_t)nS * sizeof(WideSum) + 15) & ~(size_t)15); }
   __host__ __device__ size_t row_off() const { return dec_off() + 64; }
   __host__ __device__ size_t scale_off() const { return row_off() + 128; }
-  __host__ __device__ size_t hist_off() const { return scale_off() + 128; }
-  __host__ __device__ size_t group_off() const { return hist_off() + (size_t)nS * kWideBins * sizeof(float); }
-  __host__ __device__ size_t cand_off() const { return group_off() + (size_t)nS * kWideGroups * sizeof(uint16_t); }
-  __host__ __device__ size_t touch_off() const { return cand_off() + (size_t)nS * cand_cap() * 12; }
-  // Touched tokens the rest of the row's workspace holds (a float64 value and a 16-bit key each).
-  __host__ __device__ int64_t touch_cap() const {
-    const int64_t left = (int64_t)(ws_stride(V) * sizeof(double)) - (int64_t)touch_off();
-    return left < 16 ? 0 : (left / 10) & ~(int64_t)7;
+  __host__ __device__ size_t kind_off() const { return scale_off() + 128; }
+  __host__ __device__ size_t cand_off() const { return kind_off() + (size_t)nS * kWideBins * sizeof(float); }
+  template <bool TOP>
+  __device__ __forceinline__ size_t touch_off() const {
+    return TOP ? kind_off() + (size_t)nS * kWideGroups * sizeof(uint16_t) : cand_off() + (size_t)nS * cand_cap() * 12;
+  }
+  // Touched tokens it holds: a float64 value and, in a top-k row, a 16-bit key each.
+  template <bool TOP>
+  __device__ __forceinline__ int touch_cap() const {
+    const uint32_t left = (uint32_t)(ws_stride(V) * sizeof(double) - touch_off<TOP>());  // positive from kWideMinVocab on
+    return (int)((left / (TOP ? 10u : 8u)) & ~7u);
   }
   __device__ __forceinline__ WideRec* rec(char* w) const { return (WideRec*)w; }
   __device__ __forceinline__ WideSum* sum(char* w) const { return (WideSum*)(w + sum_off()); }
   __device__ __forceinline__ WideDec* dec(char* w) const { return (WideDec*)(w + dec_off()); }
   __device__ __forceinline__ WideRow* row(char* w) const { return (WideRow*)(w + row_off()); }
   __device__ __forceinline__ double* scale(char* w) const { return (double*)(w + scale_off()); }  // each slice's exp((m - M) / T)
-  __device__ __forceinline__ float* hist(char* w) const { return (float*)(w + hist_off()); }
-  __device__ __forceinline__ uint16_t* group(char* w) const { return (uint16_t*)(w + group_off()); }
+  __device__ __forceinline__ float* hist(char* w) const { return (float*)(w + kind_off()); }
+  __device__ __forceinline__ uint16_t* group(char* w) const { return (uint16_t*)(w + kind_off()); }
   // Listed tokens of slice s: values, then token ids.
   __device__ __forceinline__ double* cand_v(char* w, int s) const { return (double*)(w + cand_off()) + (size_t)s * cand_cap(); }
   __device__ __forceinline__ int32_t* cand_i(char* w, int s) const {
     return (int32_t*)(w + cand_off() + (size_t)nS * cand_cap() * 8) + (size_t)s * cand_cap();
   }
-  __device__ __forceinline__ double* tv(char* w) const { return (double*)(w + touch_off()); }
-  __device__ __forceinline__ uint16_t* tk(char* w) const { return (uint16_t*)(w + touch_off() + (size_t)touch_cap() * 8); }
+  template <bool TOP>
+  __device__ __forceinline__ double* tv(char* w) const { return (double*)(w + touch_off<TOP>()); }
+  __device__ __forceinline__ uint16_t* tk(char* w) const {
+    return (uint16_t*)(w + touch_off<true>() + (size_t)touch_cap<true>() * 8);
+  }
 };
 
 // Vocabularies the path takes: below it a row fits few slices, and the
@@ -158,9 +166,11 @@ enum WideKind { kWideNone = 0, kWideGreedy = 1, kWideTopK = 2, kWideWhole = 3 };
 __device__ __forceinline__ WideKind wide_kind(const RowSpec& r, const WideLayout& L) {
   const dsr_policy_t& p = r.pol;
   if (!policy_ok(p)) return kWideNone;
-  if (r.pen_n < 0 || r.bias_n < 0 || r.pen_n + r.bias_n + kWidePrefix > L.touch_cap()) return kWideNone;
+  const bool top = p.temperature != 0.0 && p.top_k >= 1 && p.top_k < r.V;
+  if (r.pen_n < 0 || r.bias_n < 0 || r.pen_n + r.bias_n + kWidePrefix > (top ? L.touch_cap<true>() : L.touch_cap<false>()))
+    return kWideNone;
   if (p.temperature == 0.0) return kWideGreedy;
-  if (p.top_k >= 1 && p.top_k < r.V) return p.top_k <= kSplitMaxK ? kWideTopK : kWideNone;
+  if (top) return p.top_k <= kSplitMaxK ? kWideTopK : kWideNone;
   return p.temperature >= 1e-290 ? kWideWhole : kWideNone;  // 1 / T stays finite
 }
 
@@ -485,7 +495,7 @@ __global__ __launch_bounds__(kWideThreads) void k_wide_scan(Src src, int nS, int
   double tmax = -INFINITY;
   uint32_t kmin = 0xFFFFFFFFu, tn = 0u, csum = 0u;  // csum saturates: more than the limit is an error anyway
   int32_t tfirst = INT32_MAX;
-  double* tv = L.tv(ws);
+  double* tv = kind == kWideTopK ? L.tv<true>(ws) : L.tv<false>(ws);
   uint16_t* tk = L.tk(ws);
   auto raw = [&](int32_t id) -> double {
     return DT == DSR_BF16 ? (double)__uint_as_float((uint32_t)((const uint16_t*)r.logits)[id] << 16)
@@ -1058,7 +1068,7 @@ __global__ __launch_bounds__(kWideThreads) void k_wide_collect(Src src, int nS) 
   const double M = w.M;
   const int lo = s * kWideSlice, hi = lo + kWideSlice < (int)r.V ? lo + kWideSlice : (int)r.V;
   const bool touched = wide_touched(r);
-  const double* tv = L.tv(ws);
+  const double* tv = L.tv<false>(ws);
   WideRec rc;
   if (touched) rc = L.rec(ws)[s];
   float v[kWidePer];
@@ -1361,7 +1371,7 @@ __device__ __forceinline__ int wide_cut(const RowSpec& r, const WideLayout& L, c
       if (v > vk) upper = fmin(upper, v);
     };
     wide_listed(L, ws, wave, n, [&](double v, int32_t) { side(v); });
-    const double* tv = L.tv(ws);
+    const double* tv = L.tv<false>(ws);
     for (int i = t; i < (int)r.pen_n; i += kThreads) side(tv[i]);
     if (t < r.prefix_n) side(tv[r.pen_n + t]);
     for (int i = t; i < (int)r.bias_n; i += kThreads) side(tv[r.pen_n + kWidePrefix + i]);
@@ -1467,7 +1477,7 @@ __device__ __forceinline__ int64_t wide_walk(const RowSpec& r, const WideLayout&
   const bool touched = wide_touched(r);
   if (touched) {
     const WideRec rc = L.rec(ws)[s];
-    const double* tv = L.tv(ws);
+    const double* tv = L.tv<false>(ws);
     if (t < kWideSlice / 32) {
       sh.w.tbits[t] = 0u;
       sh.w.fbits[t] = 0u;
@@ -1557,7 +1567,7 @@ __device__ __forceinline__ int wide_candidates_prefix(const RowSpec& r, const Wi
     for (int i = 0; i < 8; ++i) g[i] = (w4[i >> 1] >> (16 * (i & 1))) & 0xFFFFu;
   }
   const uint16_t* tk = L.tk(ws);
-  const double* tv = L.tv(ws);
+  const double* tv = L.tv<true>(ws);
   const bool touched = wide_touched(r);
   // The thread's touched tokens, place, id and key; the first kPre history
   // entries are read once.
@@ -1693,7 +1703,7 @@ __device__ __forceinline__ int wide_candidates_exact(const RowSpec& r, const Wid
   uint32_t* tbm = (uint32_t*)t.sp;   // touched tokens
   uint32_t* cbm = (uint32_t*)t.pos;  // candidates
   uint16_t* base = (uint16_t*)t.kz;  // candidates below each word
-  const double* tv = L.tv(ws);
+  const double* tv = L.tv<true>(ws);
   const bool touched = wide_touched(r);
   auto places = [&](auto f) {  // place and id
     for (int e = tid; e < (int)r.pen_n; e += kThreads) f(e, r.pen_ids[e]);
@@ -1898,7 +1908,7 @@ __global__ __launch_bounds__(kWideThreads) void k_wide_probs(Src src, int nS) {
   }
   if (touched) {
     __syncthreads();  // after the zeros stored for these tokens above
-    const double* tv = L.tv(ws);
+    const double* tv = L.tv<false>(ws);
     wide_touched_each<kWideThreads>(r, rc.e0, rc.e1, rc.b0, rc.b1, lo, hi, [&](int at, int32_t id) {
       const double x = tv[at];
       if (!(x > -(double)INFINITY)) return;  // masked, or counted at another place: 0

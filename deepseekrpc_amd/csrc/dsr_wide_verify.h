@@ -183,7 +183,7 @@ __device__ __forceinline__ double wide_prob_at(const dsr_verify_args_t& a, const
     if (e1 > e0) at = r.pen_n + kWidePrefix + e0;
   }
   double v = -INFINITY;
-  if (at >= 0) v = W.tv(ws)[at];
+  if (at >= 0) v = W.tv<false>(ws)[at];
   else if (allowed_bit(r.allow, x)) v = load_logit(r.logits, r.dtype, x);
   return v > -(double)INFINITY && k.in(v, x) ? k.mass(v) / S : 0.0;
 }
@@ -321,7 +321,7 @@ __global__ __launch_bounds__(kWideThreads) void k_wide_residual(dsr_verify_args_
       if (in) add((double)vp[k], (double)vq[k], id);
   }
   if (touched) {
-    const double *tp = W.tv(w.wp), *tq = W.tv(w.wq);
+    const double *tp = W.tv<false>(w.wp), *tq = W.tv<false>(w.wq);
     wide_touched_each<kWideThreads>(w.p, rc.e0, rc.e1, rc.b0, rc.b1, lo, hi, [&](int at, int32_t id) { add(tp[at], tq[at], id); });
   }
   sum = wave_sum(sum);
@@ -405,7 +405,7 @@ __global__ __launch_bounds__(kThreads) void k_wide_resolve(dsr_verify_args_t a, 
     lds_barrier();  // the clear bitmaps
     if (touched) {
       const WideRec rc = W.rec(w.wp)[s];
-      const double *tp = W.tv(w.wp), *tq = W.tv(w.wq);
+      const double *tp = W.tv<false>(w.wp), *tq = W.tv<false>(w.wq);
       wide_touched_each<kThreads>(w.p, rc.e0, rc.e1, rc.b0, rc.b1, lo, hi, [&](int at, int32_t id) {
         const double x = w(tp[at], tq[at], id);
         const uint32_t bit = 1u << ((id - lo) & 31);
