@@ -1043,8 +1043,16 @@ constexpr int64_t kWideTopkVocab = 32768;
 // general one (V = 129,280): FP32 rows of mixed whole policies, 1 row 25.9 us against
 // 112, 64 rows 72 against 308, 256 rows 146 against 511; FP32 top-k 50 with
 // 2,000-token histories, 1 row 22.6 against 46.5, 64 rows 31.6 against 98.7.
+// Shorter rows than 16,384 tokens come here for a top-k or greedy alone (V =
+// 9,001, bf16 top-k rows, 32 rows: 28 us against 60).  The whole rows' six launches cost
+// more than one workgroup's general passes over so short a row (V = 9,001,
+// FP32 min-p: 256 rows 50 us against 38, 64 rows 45 against 35; top-p and
+// min-p, 1 row: 72 against 48; at 16,399, 64 rows with top-p: 65 against 155).
+constexpr int64_t kWideWholeVocab = 16384;
+
 static bool wide_path_eligible(const dsr_sample_args_t& a) {
-  return (a.dtype == DSR_BF16 || a.dtype == DSR_F32) && a.vocab >= kWideMinVocab && a.rows > 0 &&
+  return (a.dtype == DSR_BF16 || a.dtype == DSR_F32) && a.rows > 0 &&
+         a.vocab >= ((a.hints & DSR_HINT_TOPK_ALL) ? kWideMinVocab : kWideWholeVocab) &&
          (a.hints & (DSR_HINT_WHOLE_SOME | DSR_HINT_WHOLE_ALL | DSR_HINT_TOPK_ALL)) &&
          ((uintptr_t)a.workspace & 15u) == 0 &&  // its records, keys and block masses are read 16 bytes at a time
          a.rows * (int64_t)WideLayout(a.vocab).nS * kWideThreads < ((int64_t)1 << 32);
@@ -1266,7 +1274,8 @@ int32_t dsr_sample_rows_noalloc(const dsr_sample_args_t* args, void* stream) {
 // general path.
 static bool wide_verify_eligible(const dsr_verify_args_t& a) {
   const int64_t n = a.rows * (2 * (int64_t)a.K + 1);
-  return (a.dtype == DSR_BF16 || a.dtype == DSR_F32) && a.vocab >= kWideMinVocab && ((uintptr_t)a.workspace & 15u) == 0 &&
+  return (a.dtype == DSR_BF16 || a.dtype == DSR_F32) && ((uintptr_t)a.workspace & 15u) == 0 &&
+         a.vocab >= ((a.hints & DSR_HINT_TOPK_ALL) ? kWideMinVocab : kWideWholeVocab) &&  // as for sampled rows
          n * WideLayout(a.vocab).nS * kWideThreads < ((int64_t)1 << 32);
 }
 

@@ -100,8 +100,9 @@ def test_penalised_and_biased_rows(V, dtype, family):
     allowed = rng.random((B, V)) < 0.9
     u = rng.random(B)
     flags = sample(x, pols, u, dtype, 3, counts, gens, biases, allowed)
-    # A row with fewer 16-token groups than its top-k goes to the general path.
-    on = np.array([p.get("top_k", 0) <= V // 16 for p in pols])
+    # A row with fewer 16-token groups than its top-k may go to the general path; so do short rows of batches that
+    # are not all top-k or greedy, for which that path is the faster one.
+    on = np.array([p.get("top_k", 0) <= V // 16 and (V >= 16384 or family == "topk") for p in pols])
     assert (flags & N.FLAG_SPLIT).astype(bool)[on].all(), [hex(int(f)) for f in flags]
 
 

@@ -12,7 +12,7 @@ from test_gpu_wide import sample
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("V,n", [(8192, 900), (40000, 4000)])
+@pytest.mark.parametrize("V,n", [(16384, 1800), (40000, 4000)])
 def test_a_cut_among_tiny_masses(V, n):
     """One token of nearly all the mass and n of about 1e-12: the boundary lies among those."""
     rng = np.random.default_rng(V)

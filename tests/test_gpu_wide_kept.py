@@ -15,7 +15,7 @@ pytestmark = pytest.mark.gpu
 
 
 # The last word, vector and slice whole or cut short; enough workgroups that their waves start apart.
-@pytest.mark.parametrize("V,rows", [(8192, 300), (8193, 200), (40007, 128), (129280, 64)])
+@pytest.mark.parametrize("V,rows", [(16384, 300), (16385, 200), (40007, 128), (129280, 64)])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("mask", [False, True])
 def test_every_finite_token_is_kept(V, rows, dtype, mask):

@@ -17,7 +17,7 @@ pytestmark = pytest.mark.gpu
 DEV = "cuda"
 
 
-@pytest.mark.parametrize("V", [8193, 24577, 129280])
+@pytest.mark.parametrize("V", [16385, 24577, 129280])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_slices_without_a_finite_token(V, dtype):
     rng = np.random.default_rng(V)

@@ -18,7 +18,7 @@ POLICIES = [dict(top_p=0.9), dict(temperature=0.7, top_p=0.95), dict(min_p=0.05)
 
 
 @pytest.mark.parametrize("offset", [-150.0, -80.0, 20.0, 70.0])
-@pytest.mark.parametrize("V", [8193, 40007, 129280])
+@pytest.mark.parametrize("V", [16385, 40007, 129280])
 def test_a_common_offset_keeps_the_path(V, offset):
     rng = np.random.default_rng(V + int(offset) + 1000)
     B = len(POLICIES)
@@ -33,7 +33,7 @@ def test_a_common_offset_keeps_the_path(V, offset):
     assert (flags & N.FLAG_SPLIT).all(), [hex(int(f)) for f in flags]
 
 
-@pytest.mark.parametrize("V", [8192, 24575, 129280])
+@pytest.mark.parametrize("V", [16384, 24575, 129280])
 @pytest.mark.parametrize("width,offset", [(1e-3, 2e-3), (0.05, 8.0), (30.0, -500.0)])
 def test_close_rows(V, width, offset):
     rng = np.random.default_rng(V + int(1000 * width))

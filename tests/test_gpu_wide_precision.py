@@ -16,7 +16,7 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("T", [0.7, 1.0, 1.3, 7.1])
 def test_masses_are_one_exp_of_the_ieee_quotient(T):
     rng = np.random.default_rng(int(10 * T))
-    V, B = 8192, 4
+    V, B = 16384, 4
     x = rng.uniform(-690 * T, 0, (B, V)).astype(np.float32)
     x[:, 17] = 0.0
     x[1] += np.float32(3.25)
