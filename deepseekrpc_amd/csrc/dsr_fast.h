@@ -26,7 +26,8 @@ constexpr int kHandInvalid = 6;    // invalid or fully masked logits (reported i
 // copy of the arguments (the caller's DSR_HINT_* bits are not passed on).
 constexpr uint32_t kModeDeferWhole = 1u << 8;  // top-k register kernel: leave whole rows untouched
 constexpr uint32_t kModeOnlyWhole = 1u << 9;   // full-vocabulary kernel: decide whole rows only
-constexpr uint32_t kModeGreedyDone = 1u << 10;  // full-vocabulary kernel: greedy rows are decided unless left to it
+constexpr uint32_t kModeGreedyDone = 1u << 11;  // full-vocabulary kernel: greedy rows are decided unless left to it
+constexpr uint32_t kModeLongFirst = 1u << 10;  // full-vocabulary kernel: the rows it samples start first
 
 // A whole row: sampled (0 < T <= 100) without a top-k the register kernel
 // takes, so its filters keep the whole vocabulary or a top-k above 1024.  In

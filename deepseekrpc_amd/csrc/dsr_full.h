@@ -1083,18 +1083,12 @@ __device__ __forceinline__ int full_sample_row(const dsr_sample_args_t& a, int64
   return sh.bc_i[2] ? kHandCapacity : 0;  // unreachable: thr lies inside the chunk found above
 }
 
-
 // Greedy rows with a history, in a launch of their own ahead of the
-// full-vocabulary kernel when a batch has more rows than the chip has CUs.  A
+// full-vocabulary kernel (k_greedy_bf16) where a batch has many of them.  A
 // greedy row needs no key counts: 22 KB of LDS and 64 registers let two rows
 // share a CU, so one's loads hide the other's steps, where the
-// full-vocabulary kernel's 160 KB hold one; and the sampled rows, left alone
-// in that kernel, no longer wait in launch order behind greedy ones (the
-// workgroups go to XCDs and shader engines in turn, so a batch of alternating
-// rows kept the sampled ones on half of them).
-// 1,024 rows of 129,280 with 16,384-token histories, greedy and nearly flat
-// top-p rows in turn: 300 us with this launch and rotated rows (spread_row),
-// 378 with rotated rows alone, 459 with neither.
+// full-vocabulary kernel's 160 KB hold one.  Returns false, with nothing
+// written, for a row that full_sample_row must decide.
 constexpr int32_t kGreedyLeft = INT32_MIN;  // out_status of a greedy row left to the full-vocabulary kernel
 
 struct GreedyShared {

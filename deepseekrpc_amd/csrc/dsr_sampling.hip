@@ -236,22 +236,78 @@ struct FullKernelShared {
   };
 };
 
-// The row of workgroup b.  Workgroups go to the eight XCDs in turn, and in each
-// to its four shader engines in turn, whatever those still hold: in a batch
-// whose rows alternate in kind, the costly rows would all meet on the same
-// engines.  So group k of 32 workgroups takes its 32 rows rotated by 11 k,
-// which keeps moving every bit of the row's number over the engines.
-__device__ __forceinline__ int64_t spread_row(uint32_t b, uint32_t rows) {
-  return (b | 31u) < rows ? (int64_t)((b & ~31u) | ((b + 11u * (b >> 5)) & 31u)) : (int64_t)b;
+// The row of workgroup b in a batch of several rounds over the chip: the rows
+// this kernel samples come first, in order, then the others.  The kernel holds
+// one row on a CU, and its greedy rows take a quarter of a sampled one's time;
+// workgroups start in order, handed to the XCDs and their shader engines in
+// turn, so the long rows started first spread evenly over the CUs and the short
+// ones fill in behind them.  In the batch's own order they meet as they come (of
+// alternating rows the sampled ones all on half of the engines).  Every
+// workgroup reads all rows' policies (2 us); rows <= kLongRows.
+constexpr int kLongRows = 4 * kThreads;
+
+struct LongScratch {
+  unsigned long long mask[kLongRows / 64];  // the long ones of each 64 rows
+};
+
+// Lane l's 64 rows (64 l .. 64 l + 63), in every wave: the long ones; `all` of them.
+template <class Long>
+__device__ __forceinline__ unsigned long long long_rows(uint32_t rows, LongScratch& sh, Long is_long, uint32_t& all) {
+  constexpr int kParts = kLongRows / kThreads;
+  static_assert(kLongRows / 64 == 64, "a group of rows per lane");
+  bool f[kParts];
+#pragma unroll
+  for (int q = 0; q < kParts; ++q) {
+    const uint32_t r = (uint32_t)q * kThreads + threadIdx.x;
+    f[q] = r < rows && is_long(r);
+  }
+#pragma unroll
+  for (int q = 0; q < kParts; ++q) {
+    const unsigned long long m = __ballot(f[q]);
+    if (lane_id() == 0) sh.mask[q * kWaves + wave_id()] = m;
+  }
+  lds_barrier();
+  const unsigned long long m = sh.mask[lane_id()];
+  all = wave_reduce_dpp((uint32_t)__popcll(m), OpSum());
+  return m;
+}
+
+// `all`: the long rows of the batch.
+template <class Long>
+__device__ __forceinline__ int64_t long_first(uint32_t b, uint32_t rows, LongScratch& sh, uint32_t& all, Long is_long) {
+  unsigned long long m = long_rows(rows, sh, is_long, all);
+  const int l = lane_id();
+  const int valid = min(max((int)rows - 64 * l, 0), 64);
+  uint32_t want = b;
+  if (b >= all) {  // uniform
+    want = b - all;
+    m = ~m & (valid == 64 ? ~0ull : (1ull << valid) - 1ull);
+  }
+  const uint32_t n = (uint32_t)__popcll(m), incl = wave_scan_dpp(n);
+  const int g = __ffsll((long long)__ballot(incl > want)) - 1;  // b < rows: some lane passes it
+  const unsigned long long gm = (unsigned long long)lane_value((long long)m, g);
+  const uint32_t in = want - (lane_value(incl, g) - (uint32_t)__popcll(gm));
+  const bool here = ((gm >> l) & 1ull) && (uint32_t)__popcll(gm & ((1ull << l) - 1ull)) == in;
+  const int e = __ffsll((long long)__ballot(here)) - 1;
+  __syncthreads();  // the scratch is free
+  return 64 * (int64_t)g + e;
 }
 
 template <bool RNG>
 __global__ __launch_bounds__(kThreads) void k_sample_bf16_full(dsr_sample_args_t a) {
   __shared__ FullKernelShared sh;
-  const int64_t row = spread_row(blockIdx.x, gridDim.x);
+  const bool only_whole = a.hints & kModeOnlyWhole;
+  int64_t row = blockIdx.x;
+  if (a.hints & kModeLongFirst) {
+    uint32_t all;
+    row = long_first(blockIdx.x, gridDim.x, *(LongScratch*)&sh, all, [&](uint32_t r) {
+      const dsr_policy_t& p = a.policy[r];
+      return only_whole ? whole_row(p.temperature, p.top_k, a.vocab) : p.temperature != 0.0;
+    });
+  }
   // After the top-k register kernel: only the rows it left (uniform; read
   // before the row's loads are issued, so other rows cost no HBM traffic).
-  if ((a.hints & kModeOnlyWhole) && !whole_row(a.policy[row].temperature, a.policy[row].top_k, a.vocab)) return;
+  if (only_whole && !whole_row(a.policy[row].temperature, a.policy[row].top_k, a.vocab)) return;
   if ((a.hints & kModeGreedyDone) && a.policy[row].temperature == 0.0 && a.out_status[row] != kGreedyLeft) return;
   const int why = full_sample_row<RNG>(a, row, sh.f);
   if (why == 0) return;
@@ -264,13 +320,25 @@ __global__ __launch_bounds__(kThreads) void k_sample_bf16_full(dsr_sample_args_t
   finish_row<RNG>(a, row, W, a.vocab, st, d, flags, sh.g);
 }
 
+// Whether a batch's greedy rows are worth a launch of their own ahead of the
+// full-vocabulary kernel: it decides 512 of them in 0.45 of a sampled row's
+// time (few of them in 0.2), where that kernel takes 0.35 of it for each, but there they also
+// fill the CUs that its last round of sampled rows leaves idle (counted at 0.7).
+// 1,024 rows, half of them greedy: 60 us and 240, against 336 in one launch.
+__device__ __forceinline__ bool greedy_apart(uint32_t rows, uint32_t greedy) {
+  const uint32_t idle = (256u - (rows - greedy) % 256u) % 256u;
+  return 0.35f / 256.0f * ((float)greedy - 2.0f * (float)idle) > fmaxf(0.2f, 0.45f / 512.0f * (float)greedy) + 0.04f;
+}
+
 template <bool RNG>
 __global__ __launch_bounds__(kThreads, 8) void k_greedy_bf16(dsr_sample_args_t a) {
   __shared__ GreedyShared sh;
-  const int64_t row = spread_row(blockIdx.x, gridDim.x);
-  const dsr_policy_t pol = a.policy[row];
-  if (!(pol.temperature == 0.0)) return;
-  if (!greedy_row<RNG>(a, row, pol, sh) && threadIdx.x == 0) a.out_status[row] = kGreedyLeft;
+  uint32_t greedy;
+  const int64_t row = long_first(blockIdx.x, gridDim.x, *(LongScratch*)&sh, greedy,
+                                 [&](uint32_t r) { return a.policy[r].temperature == 0.0; });
+  if (blockIdx.x >= greedy) return;
+  if (!(greedy_apart(gridDim.x, greedy) && greedy_row<RNG>(a, row, a.policy[row], sh)) && threadIdx.x == 0)
+    a.out_status[row] = kGreedyLeft;
 }
 
 // Sliced path, step three (dsr_wide.h): one workgroup finishes a row from
@@ -1125,9 +1193,13 @@ size_t dsr_verify_workspace_bytes(int64_t rows, int32_t K, int64_t vocab) {
   return verify_ws_bytes(rows, K, vocab);
 }
 
+constexpr int64_t kFullRows = 256;  // CUs: the full-vocabulary kernel holds one row on each
+// Smaller batches hold too few greedy rows for a launch of their own (see
+// greedy_apart), which takes 5 us also where it leaves them.
+constexpr int64_t kGreedyRows = 768;
+
 // The DSR_HINT_* bits a caller may set; any other bit is rejected, so the
 // field can take new meanings later without an ABI change.
-constexpr int64_t kFullRows = 256;  // CUs: the full-vocabulary kernel holds one row on each
 static constexpr uint32_t kHintBits = DSR_HINT_WHOLE_SOME | DSR_HINT_WHOLE_ALL | DSR_HINT_VERIFY_FAST | DSR_HINT_TOPK_ALL;
 
 static bool dtype_ok(int32_t d) { return d == DSR_BF16 || d == DSR_F32 || d == DSR_F64; }
@@ -1172,6 +1244,9 @@ static int32_t sample_rows(const dsr_sample_args_t* args, const dsr_head_part_t*
     else hipLaunchKernelGGL(k_sample_bf16_full<false>, grid, dim3(kThreads), 0, s, k);
   };
   const bool wide = wide_path_eligible(a);
+  // Rows of several kinds in more than one round over the CUs: see long_first.
+  const uint32_t long_mode = a.rows > kFullRows && a.rows <= kLongRows && (a.hints & DSR_HINT_WHOLE_SOME) &&
+                             !(a.hints & DSR_HINT_WHOLE_ALL) ? kModeLongFirst : 0u;
   if (fast_path_eligible(a)) {
     // A bf16 batch with no history or bias: whole rows (no top-k register
     // cut) go to the full-vocabulary kernel when the caller says it has some.
@@ -1179,7 +1254,7 @@ static int32_t sample_rows(const dsr_sample_args_t* args, const dsr_head_part_t*
       launch_full(0u);
     } else if (a.hints & DSR_HINT_WHOLE_SOME) {
       launch_fast(kModeDeferWhole);
-      launch_full(kModeOnlyWhole);
+      launch_full(kModeOnlyWhole | long_mode);
     } else {
       launch_fast(0u);
     }
@@ -1189,13 +1264,12 @@ static int32_t sample_rows(const dsr_sample_args_t* args, const dsr_head_part_t*
     // on the sliced path; 1 row: 68 against 72).  It has no top-k cut, and
     // the general path takes about 1 ms for such rows: batches of top-k rows
     // go to the sliced path (64 rows, top-k 50: 32 us).
-    // Batches of several rounds with greedy rows among them (WHOLE_SOME): see greedy_row.
-    if (a.rows > kFullRows && a.pen_off && (a.hints & DSR_HINT_WHOLE_SOME) && !(a.hints & DSR_HINT_WHOLE_ALL)) {
-      if (a.rng_state) hipLaunchKernelGGL(k_greedy_bf16<true>, dim3((unsigned)a.rows), dim3(kThreads), 0, s, a);
-      else hipLaunchKernelGGL(k_greedy_bf16<false>, dim3((unsigned)a.rows), dim3(kThreads), 0, s, a);
-      launch_full(kModeGreedyDone);
+    if (long_mode && a.pen_off && a.rows >= kGreedyRows) {
+      if (a.rng_state) hipLaunchKernelGGL(k_greedy_bf16<true>, grid, dim3(kThreads), 0, s, a);
+      else hipLaunchKernelGGL(k_greedy_bf16<false>, grid, dim3(kThreads), 0, s, a);
+      launch_full(long_mode | kModeGreedyDone);
     } else {
-      launch_full(0u);
+      launch_full(long_mode);
     }
   } else if (f32_path_eligible(a) && !(wide && !parts && a.vocab >= kWideTopkVocab && a.rows * WideLayout(a.vocab).nS <= kWideTopkSlices)) {
     if (a.out_probs_f32 || a.out_probs_f64) {
