@@ -958,16 +958,27 @@ __device__ __forceinline__ int full_sample_row(const dsr_sample_args_t& a, int64
     // (no top-k on this path).
     fast_clear_outputs(a, row);
     const double Sd = (double)Sk * 0x1p-45;
+    // The row's outputs as addresses of their own, and four tokens at a time:
+    // with the arguments read at every store, from spilled scalars, 6 rows of
+    // 129,280 with FP32 probabilities take 145 us, with these 131.
+    float* const o32 = a.out_probs_f32 ? a.out_probs_f32 + row * a.probs_ld : nullptr;
+    double* const o64 = a.out_probs_f64 ? a.out_probs_f64 + row * a.probs_ld : nullptr;
+    uint32_t* const okb = a.out_kept_bits ? a.out_kept_bits + row * a.kept_ld : nullptr;
+    auto put = [&](long long i, double p) {
+      if (o32) o32[i] = (float)p;
+      if (o64) o64[i] = p;
+      if (okb) atomicOr(&okb[i >> 5], 1u << (i & 31));
+    };
 #pragma unroll
     for (int j = 0; j < kFastChunks; ++j) {
       const uint32_t c = (uint32_t)wave * CW + (uint32_t)j * 64u + (uint32_t)lane;
-#pragma unroll 1
+#pragma unroll 4
       for (int e = 0; e < 8; ++e) {
         const uint32_t k = key_at_rt(d[j], e);
         if (k > kKeyNegInf) {
           const long long idx = 8ll * c + e;
           const bool kept = L == 0u || k > L || (k == L && keep > 0 && (!split || idx <= cut_idx));
-          fast_scatter(a, row, idx, kept ? mass_of(bf16_key_value(k)) / Sd : 0.0);
+          put(idx, kept ? mass_of(bf16_key_value(k)) / Sd : 0.0);
         }
       }
     }
@@ -977,7 +988,7 @@ __device__ __forceinline__ int full_sample_row(const dsr_sample_args_t& a, int64
       const long long pk = Wp[e];
       const int32_t id = a.pen_ids[o0 + e];
       const double p = pen_kept((uint32_t)((unsigned long long)pk >> 48), id) ? mass_of(v) / Sd : 0.0;
-      fast_scatter(a, row, id, p);
+      put(id, p);
     }
   }
   if (!has_draws<RNG>(a)) {
