@@ -82,8 +82,8 @@ WORKLOADS = {
 }
 
 # Name prefix of a workload's committed profile summaries when it is not its first kernel's.
-PROFILE_PREFIX = {"c4": "k_verify", "c1": "k_sample_f32", "propose": "k_sample_f32", "seed": "k_sample_f32",
-                  "step": "k_sample_f32",
+PROFILE_PREFIX = {"c4": "k_verify", "c1": "k_wide", "propose": "k_wide", "seed": "k_wide", "step": "k_wide",
+                  "c5": "k_sample_bf16_full",
                   "head": "k_vocab_head", "headk": "k_vocab_head"}
 
 DESCRIPTIONS = {
