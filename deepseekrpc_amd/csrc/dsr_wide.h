@@ -32,14 +32,15 @@
 //                   and that slice's tokens in index order.
 //   k_wide_probs    whole rows whose probabilities are asked for.
 //
-// What bounds them, at V = 129,280: the scan of top-k rows a copy's rate (64
-// bf16 rows with 4,096-token histories 12.4 us), of whole rows the float64
-// exps and LDS atomics (23 us); the bracket two round trips to memory (6 us); the
-// collect its second read of the row (32 FP32 rows 14.6 us); the finishing
-// workgroups their chains of dependent reductions (top-k 16 us, draw 24 us);
-// the probabilities their stores (15 us).  Before it, one workgroup per row:
-// 64 bf16 rows, top-k 50, 4,096-token histories 953 us, now 28; 32 FP32 rows
-// of mixed whole policies with distributions 297, now 76.
+// What bounds them, at V = 129,280 (64 bf16 rows, top-k 50, 4,096-token
+// histories, and 32 FP32 rows of mixed whole policies with distributions): the
+// scan of top-k rows a copy's rate (12.6 us), of whole rows the float64 exps
+// and LDS atomics (13.3 us); the bracket two round trips to memory (8.1 us);
+// the collect its second read of the row (10.9 us); the finishing workgroups
+// their chains of dependent reductions (top-k 15.5 us, draw 23.8 us); the
+// probabilities their stores (14.7 us).  Before it, one workgroup per row took
+// 1,013 us for the first, now 28; the split path 297 for the second, more
+// (426 to 444) where it handed rows over, now 70.
 //
 // Bin masses only bracket a boundary (they carry 36-bit fixed point and
 // FP32 rounding, and the bracket allows for both); every decision is made

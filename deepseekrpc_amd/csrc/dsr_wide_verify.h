@@ -24,8 +24,8 @@
 //                    8,192-token slice sums its weights
 //   k_wide_resolve   the slice that holds the crossing, in index order
 //
-// 8 requests x 4 drafts, V = 129,280, FP32: top-k 20..200 with top-p 52.8 us
-// (scan 13, dist 24, dists 4.5 with nothing to do, chain 13.5) against 730
+// 8 requests x 4 drafts, V = 129,280, FP32: top-k 20..200 with top-p 51.5 us
+// (scan 12.6, dist 23.6, dists 4.6 with nothing to do, chain 12.6) against 730
 // for a workgroup per distribution writing float64 rows and one per request
 // reading them back.  The rows of the scan are read once, at the rate of a
 // copy; the two single-workgroup steps are bound by their chains of
@@ -34,7 +34,7 @@
 // A request with a row outside the path (invalid, a top-k above 1,024, a cut
 // the listed values cannot decide) is built in full by k_verify_dists and
 // decided by general_decide, as are float64 logits and vocabularies below
-// 8,192.
+// 16,384 (8,192 where the hints say that every request is top-k or greedy).
 //
 // A call takes this path as a whole: one with a history, a bias or a mask, or
 // one whose hints say that no request takes the fast path.  With neither, the
